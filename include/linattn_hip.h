@@ -137,6 +137,10 @@ typedef struct {
  * softmax; an empty row yields zeros (the reference divides by max(l,1e-12)).
  * out: (B, Hq, Tq, D) with strides o_sb/o_sh/o_st in out_dtype (F32/BF16).
  * Work is split over the list ("split-K"); num_splits = 0 picks a split count.
+ * With num_splits = 0, calls of many queries over a contiguous bf16 cache
+ * (D = 128, bf16 q) run as tiles of queries sharing key blocks when
+ * la_sparse_attention_workspace() bytes are given (16-byte aligned); with less,
+ * but enough for the split partials, they run row by row.
  */
 typedef struct {
   const void *q;
@@ -169,8 +173,8 @@ int la_sparse_attention(const la_sparse_attn_args *a, const la_kv *kv, void *str
  * runs on until the process ends (a->workspace / ws_bytes are ignored).
  * No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  Calls whose la_sparse_attention_workspace() exceeds the
- * limit fail with LA_ERR_WORKSPACE before launching anything.  Every call on
+ * forbid hipMalloc).  Every call runs row by row; calls whose split partials
+ * exceed the limit fail with LA_ERR_WORKSPACE before launching anything.  Every call on
  * one device shares that device's array: calls that overlap in time on one
  * device (other streams, other threads) race; the partials are written whole
  * by each call, so nothing needs clearing between calls.

@@ -21,6 +21,7 @@
 
 #include "common.h"
 #include "kv_access.h"
+#include "list_tile.h"
 #include "quest_select.h"
 
 namespace la {
@@ -104,16 +105,15 @@ struct RowCtx {
   int64_t k_bh, v_bh, s_bh;  // contiguous-layout bases
 };
 
-// Decodes the row of this workgroup and stages its split's entries in LDS:
+// Decodes row r and stages the entries of its part `split` in LDS:
 // the logical first token (for masking; -1 = skip) and, for a paged cache,
 // the pool row of that token, so a token costs no page-table lookup.  The
 // caller synchronises before reading the staged entries.
 template <int G, bool PAGED>
-__device__ __forceinline__ RowCtx stage_row(const AttnKP &p, int32_t *s_tok0, int32_t *s_phys) {
+__device__ __forceinline__ RowCtx stage_row(const AttnKP &p, int64_t r, int64_t split,
+                                            int32_t *s_tok0, int32_t *s_phys) {
   RowCtx rc;
   const int tid = threadIdx.x;
-  const int64_t r = blockIdx.y;
-  const int64_t split = blockIdx.x;
   rc.t = r % p.Tq;
   const int64_t ih = (r / p.Tq) % p.ids_heads;
   rc.b = r / (p.Tq * p.ids_heads);
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(SA_NT) void sparse_attn_kernel(AttnKP p) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int c = lane % LPR;     // chunk of D this lane owns
   const int slot = lane / LPR;  // row slot within the wave
-  const RowCtx rc = stage_row<G, PAGED>(p, s_tok0, s_phys);
+  const RowCtx rc = stage_row<G, PAGED>(p, blockIdx.y, blockIdx.x, s_tok0, s_phys);
   const int32_t lim32 = (int32_t)min(rc.lim, (int64_t)0x7fffffff);
 
   // q chunk of this lane for the G heads, pre-scaled into the log2 domain.
@@ -764,11 +764,77 @@ __global__ __launch_bounds__(SA_NT, G <= 4 ? 4 : 2) void sparse_attn_mfma_kernel
   __shared__ int32_t s_tok0[SA_MAX_EPS];
   __shared__ int32_t s_phys[PAGED ? SA_MAX_EPS : 1];
   __shared__ MfmaLds<KT, G, SA_NW> L;
-  const RowCtx rc = stage_row<G, PAGED>(p, s_tok0, s_phys);
+  const RowCtx rc = stage_row<G, PAGED>(p, blockIdx.y, blockIdx.x, s_tok0, s_phys);
   mfma_attend<KT, G, PAGED, U16, SA_NW>(p, rc, s_tok0, s_phys, L);
   finish_row<G, 128, SA_NW>(p, rc, blockIdx.y, blockIdx.x, L.acc, L.m, L.l);
 }
 
+// The rows a tiled call (list_tile.hip) left to be attended row by row: a
+// workgroup looks at rows_per_wg rows and attends those the gate marks, part
+// by part of SA_MAX_EPS list entries (p.splits), the parts merged in
+// registers.  Usually no row is marked and the launch is the look alone.
+template <int G>
+__global__ __launch_bounds__(SA_NT, G <= 4 ? 4 : 2) void sparse_attn_gated_kernel(AttnKP p,
+                                                                                  ListTileGate gt,
+                                                                                  int64_t R,
+                                                                                  int32_t rows_per_wg) {
+  __shared__ int32_t s_tok0[SA_MAX_EPS];
+  __shared__ MfmaLds<LA_BF16, G, SA_NW> L;
+  constexpr int D = 128, NI = (G * D + SA_NT - 1) / SA_NT;
+  // lane i of every wave looks at row r0 + i (rows_per_wg <= 64)
+  const int64_t r0 = (int64_t)blockIdx.x * rows_per_wg;
+  const int lane = threadIdx.x & 63;
+  bool mine = false;
+  if (lane < rows_per_wg && r0 + lane < R) {
+    const int64_t r = r0 + lane;
+    const int64_t t = r % p.Tq, ih = (r / p.Tq) % p.ids_heads, b = r / (p.Tq * p.ids_heads);
+    const int64_t h0 = p.ids_heads == p.Hkv ? ih * G : ih;
+    mine = gt.dup[b * gt.m_sb + ih * gt.m_sh + t * gt.m_st] != 0 || gt.tile_left(b, h0, t);
+    for (int g = 0; g < G && !mine; ++g) mine = gt.rgate[(b * p.Hq + h0 + g) * p.Tq + t] != 0;
+  }
+  for (uint64_t todo = __ballot(mine); todo; todo &= todo - 1) {
+    const int64_t r = r0 + __ffsll((unsigned long long)todo) - 1;
+    float M[NI], S[NI], A[NI];
+#pragma unroll
+    for (int x = 0; x < NI; ++x) {
+      M[x] = __int_as_float(0xff800000);
+      S[x] = A[x] = 0.f;
+    }
+    RowCtx rc;
+    for (int64_t part = 0; part < p.splits; ++part) {
+      rc = stage_row<G, false>(p, r, part, s_tok0, nullptr);
+      mfma_attend<LA_BF16, G, false, false, SA_NW>(p, rc, s_tok0, nullptr, L);
+#pragma unroll
+      for (int x = 0; x < NI; ++x) {
+        const int i = threadIdx.x + SA_NT * x;
+        if (i >= G * D) break;
+        const int g = i / D, d = i % D;
+        float mn = M[x];
+#pragma unroll
+        for (int y = 0; y < SA_NW; ++y) mn = fmaxf(mn, L.m[y][g]);
+        const float mu = mn == __int_as_float(0xff800000) ? 0.f : mn;
+        const float old = fast_exp2(M[x] - mu);
+        S[x] *= old;
+        A[x] *= old;
+#pragma unroll
+        for (int y = 0; y < SA_NW; ++y) {
+          const float sc = fast_exp2(L.m[y][g] - mu);
+          S[x] += L.l[y][g] * sc;
+          A[x] += L.acc[y][g][d] * sc;
+        }
+        M[x] = mn;
+      }
+      __syncthreads();  // the states are read before the next part's fill
+    }
+#pragma unroll
+    for (int x = 0; x < NI; ++x) {
+      const int i = threadIdx.x + SA_NT * x;
+      if (i >= G * D) break;
+      store_from_f32(p.out, rc.b * p.o_sb + (rc.h0 + i / D) * p.o_sh + rc.t * p.o_st + i % D, p.out_dt,
+                     S[x] > 0.f ? A[x] / S[x] : 0.f);
+    }
+  }
+}
 
 // ---------------------------------------------- fused Quest decode ----
 // One workgroup of eight waves per (b, KV head) with one query per sequence:
@@ -865,27 +931,81 @@ __global__ __launch_bounds__(QD_NT, 4) void quest_decode_fused_kernel(QsKP a, At
   finish_row<G, 128, QD_NW>(p, rc, row, 0, L.u.att.acc, L.u.att.m, L.u.att.l);
 }
 
-// Merge the split partials of one (row, head): one workgroup, D threads.
-__global__ __launch_bounds__(256) void sparse_attn_combine(AttnKP p, int64_t G, int64_t D) {
-  const int64_t rg = blockIdx.x;
+// Merge the split partials of the (row, head)s: 32 lanes each, eight per
+// workgroup, a lane D / 32 neighbouring dims.  Latency-bound, so four splits'
+// maxima, sums and values are read at once: one memory round trip (a merge of
+// 32768 rows of two parts took 27 us with one workgroup per row and a round
+// trip per split, 9 us like this).  TILES: the parts of list_tile.hip, whose
+// left-out tiles hold none and whose results are marked where not finite.
+template <int D, bool TILES>
+__global__ __launch_bounds__(256) void sparse_attn_combine(AttnKP p, int64_t G, int64_t RG,
+                                                           ListTileGate gt) {
+  constexpr int DL = D / 32, NS = 4;
+  const int c = threadIdx.x & 31;
+  const int64_t rg = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
+  if (rg >= RG) return;
   const int64_t r = rg / G, g = rg % G;
   const int64_t t = r % p.Tq;
   const int64_t ih = (r / p.Tq) % p.ids_heads;
   const int64_t b = r / (p.Tq * p.ids_heads);
   const int64_t h = ((p.ids_heads == p.Hkv) ? ih * G : ih) + g;
   const float *ml = p.ws_ml + rg * p.splits * 2;
-  float M = __int_as_float(0xff800000);
-  for (int64_t s = 0; s < p.splits; ++s) M = fmaxf(M, ml[2 * s]);
-  const float Mu = (M == __int_as_float(0xff800000)) ? 0.f : M;
-  for (int64_t d = threadIdx.x; d < D; d += blockDim.x) {
-    float L = 0.f, A = 0.f;
-    for (int64_t s = 0; s < p.splits; ++s) {
-      const float sc = fast_exp2(ml[2 * s] - Mu);
-      L += ml[2 * s + 1] * sc;
-      A += p.ws_acc[(rg * p.splits + s) * D + d] * sc;
+  const float *pa = p.ws_acc + rg * p.splits * D + DL * c;
+  const float NEG_INF = __int_as_float(0xff800000);
+  bool left = false;
+  if constexpr (TILES) left = gt.tile_left(b, h, t);
+  float M = NEG_INF, L = 0.f, A[DL];
+#pragma unroll
+  for (int e = 0; e < DL; ++e) A[e] = 0.f;
+  const int ns = (int)p.splits;
+  for (int s0 = 0; s0 < ns; s0 += NS) {
+    float m[NS], l[NS], y[NS][DL];
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      const int s = min(s0 + u, ns - 1);
+      m[u] = ml[2 * s];
+      l[u] = ml[2 * s + 1];
+#pragma unroll
+      for (int e = 0; e < DL; ++e) y[u][e] = pa[(int64_t)s * D + e];
     }
-    const float o = L > 0.f ? A / L : 0.f;
-    store_from_f32(p.out, b * p.o_sb + h * p.o_sh + t * p.o_st + d, p.out_dt, o);
+    float mn = M;
+#pragma unroll
+    for (int u = 0; u < NS; ++u) mn = s0 + u < ns ? fmaxf(mn, m[u]) : mn;
+    const float mu = mn == NEG_INF ? 0.f : mn;
+    const float old = fast_exp2(M - mu);
+    L *= old;
+#pragma unroll
+    for (int e = 0; e < DL; ++e) A[e] *= old;
+#pragma unroll
+    for (int u = 0; u < NS; ++u) {
+      if (s0 + u >= ns) break;
+      const float f = fast_exp2(m[u] - mu);
+      L += l[u] * f;
+#pragma unroll
+      for (int e = 0; e < DL; ++e) A[e] = __builtin_fmaf(y[u][e], f, A[e]);
+    }
+    M = mn;
+  }
+  if (left) return;
+  float v[DL];
+#pragma unroll
+  for (int e = 0; e < DL; ++e) v[e] = L > 0.f ? A[e] / L : 0.f;
+  if constexpr (TILES) {
+    bool fin = L < __int_as_float(0x7f800000);
+#pragma unroll
+    for (int e = 0; e < DL; ++e) fin = fin && fabsf(A[e]) < __int_as_float(0x7f800000);
+    const uint64_t bad = __ballot(!fin) >> (threadIdx.x & 32);  // this row's 32 lanes
+    if (c == 0) gt.rgate[(b * p.Hq + h) * p.Tq + t] = (uint32_t)bad != 0;
+  }
+  const int64_t o = b * p.o_sb + h * p.o_sh + t * p.o_st + DL * c;
+  if (p.out_dt == LA_BF16 && ((uintptr_t)p.out + 2 * o) % 4 == 0) {
+#pragma unroll
+    for (int e = 0; e < DL; e += 2)
+      *(uint32_t *)((uint16_t *)p.out + o + e) =
+          (uint32_t)f32_to_bf16_bits(v[e]) | ((uint32_t)f32_to_bf16_bits(v[e + 1]) << 16);
+  } else {
+#pragma unroll
+    for (int e = 0; e < DL; ++e) store_from_f32(p.out, o + e, p.out_dt, v[e]);
   }
 }
 
@@ -920,7 +1040,8 @@ static int launch_attn(const AttnKP &p, hipStream_t st) {
     sparse_attn_kernel<KT, D, G, UNR, PAGED><<<grid, SA_NT, 0, st>>>(p);
   LA_LAUNCHED();
   if (p.splits > 1) {
-    sparse_attn_combine<<<dim3((unsigned)(p.B * p.ids_heads * p.Tq * G)), D, 0, st>>>(p, G, D);
+    const int64_t RG = p.B * p.ids_heads * p.Tq * G;
+    sparse_attn_combine<D, false><<<dim3((unsigned)ceil_div(RG, 8)), 256, 0, st>>>(p, G, RG, ListTileGate{});
     LA_LAUNCHED();
   }
   return LA_OK;
@@ -957,7 +1078,8 @@ static int dispatch_d(const AttnKP &p, int64_t D, int64_t G, hipStream_t st) {
 
 struct Plan {
   int64_t G, R, splits, eps;
-  size_t ws;
+  size_t ws;          // row kernels: split partials
+  ListTilePlan tile;  // many queries with lists of their own: tiles
 };
 
 static int plan_attn(const la_sparse_attn_args *a, const la_kv *kv, Plan &pl) {
@@ -1007,6 +1129,7 @@ static int plan_attn(const la_sparse_attn_args *a, const la_kv *kv, Plan &pl) {
   splits = ceil_div(a->N, pl.eps);
   pl.splits = splits;
   pl.ws = splits > 1 ? (size_t)(pl.R * pl.G * splits) * (size_t)(a->D + 2) * sizeof(float) : 0;
+  pl.tile = list_tile_plan(a, kv);
   return LA_OK;
 }
 
@@ -1017,14 +1140,12 @@ using namespace la;
 extern "C" size_t la_sparse_attention_workspace(const la_sparse_attn_args *a, const la_kv *kv) {
   Plan pl{};
   if (plan_attn(a, kv, pl) != LA_OK) return 0;
-  return pl.ws;
+  return std::max(pl.ws, pl.tile.use ? pl.tile.bytes : 0);
 }
 
 namespace la {
 
-// Launch of a planned attention with its split-K partials in `ws`.
-static int sparse_attention_run(const la_sparse_attn_args *a, const la_kv *kv, const Plan &pl,
-                                void *ws, hipStream_t st) {
+static AttnKP attn_params(const la_sparse_attn_args *a, const la_kv *kv, const Plan &pl) {
   AttnKP p{};
   p.q = a->q;
   p.out = a->out;
@@ -1058,6 +1179,44 @@ static int sparse_attention_run(const la_sparse_attn_args *a, const la_kv *kv, c
   p.causal = a->causal;
   p.staged = kv->page_table ? (kv->page_size % a->unit == 0) : 0;
   p.unit_shift = is_pow2(a->unit) ? ilog2(a->unit) : -1;
+  return p;
+}
+
+// The tiles (list_tile.hip), the merge of their parts, then the rows they
+// left.
+static int sparse_attention_tiles(const la_sparse_attn_args *a, const la_kv *kv, const Plan &pl,
+                                  void *ws, hipStream_t st) {
+  ListTileGate gate{};
+  const int rc = list_tile_launch(a, kv, pl.tile, ws, gate, st);
+  if (rc != LA_OK) return rc;
+  AttnKP p = attn_params(a, kv, pl);
+  if (pl.tile.splits > 1) {
+    p.splits = pl.tile.splits;
+    p.ws_ml = (float *)((char *)ws + pl.tile.off_ml);
+    p.ws_acc = (float *)((char *)ws + pl.tile.off_acc);
+    sparse_attn_combine<128, true><<<dim3((unsigned)ceil_div(pl.R * pl.G, 8)), 256, 0, st>>>(p, pl.G, pl.R * pl.G, gate);
+    LA_LAUNCHED();
+  }
+  p.splits = ceil_div(a->N, SA_MAX_EPS);
+  // At most 64 rows a workgroup (a lane looks at each).  Where only marked rows
+  // are left 2048 workgroups do (the look alone: 5 us, 14 us with 8192); where
+  // tiles decide, whole tiles may be left and are spread over four times as many.
+  const int32_t rpw = (int32_t)std::min<int64_t>(64, ceil_div(pl.R, pl.tile.row_cost > 0.f ? 8192 : 2048));
+  const dim3 grid((unsigned)ceil_div(pl.R, rpw));
+  switch (pl.G) {
+    case 1: sparse_attn_gated_kernel<1><<<grid, SA_NT, 0, st>>>(p, gate, pl.R, rpw); break;
+    case 2: sparse_attn_gated_kernel<2><<<grid, SA_NT, 0, st>>>(p, gate, pl.R, rpw); break;
+    case 4: sparse_attn_gated_kernel<4><<<grid, SA_NT, 0, st>>>(p, gate, pl.R, rpw); break;
+    default: sparse_attn_gated_kernel<8><<<grid, SA_NT, 0, st>>>(p, gate, pl.R, rpw); break;
+  }
+  LA_LAUNCHED();
+  return LA_OK;
+}
+
+// Launch of a planned attention with its split-K partials in `ws`.
+static int sparse_attention_run(const la_sparse_attn_args *a, const la_kv *kv, const Plan &pl,
+                                void *ws, hipStream_t st) {
+  AttnKP p = attn_params(a, kv, pl);
   if (pl.splits > 1) {
     p.ws_ml = (float *)ws;
     p.ws_acc = p.ws_ml + pl.R * pl.G * pl.splits * 2;
@@ -1106,6 +1265,9 @@ extern "C" int la_sparse_attention(const la_sparse_attn_args *a, const la_kv *kv
   Plan pl{};
   int rc = plan_attn(a, kv, pl);
   if (rc != LA_OK) return rc;
+  if (pl.tile.use && a->workspace && (uintptr_t)a->workspace % 16 == 0 &&
+      (size_t)a->ws_bytes >= pl.tile.bytes)
+    return sparse_attention_tiles(a, kv, pl, a->workspace, (hipStream_t)stream);
   if (pl.ws > 0) {
     LA_REQUIRE(a->workspace != nullptr, "sparse attention: workspace required");
     if ((size_t)a->ws_bytes < pl.ws)

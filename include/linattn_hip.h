@@ -464,8 +464,8 @@ int la_block_select(const la_block_select_args *a, void *stream);
  * q: (B, Hq, Tq, D), k: (B, Hkv, T, D) at element strides; query head h reads
  * KV head h / (Hq/Hkv).  Output: out_idx[((b*Hq + h)*Tq + t)*width + i]
  * ascending, -1 padded (width >= min(topk, blocks) + 1), out_count the number
- * kept.  Workspace: la_gate_select_workspace bytes (fp64 q, pooled keys and
- * the gate rows).  kbar (optional): the block means of k, (B, Hkv, n_kb, D)
+ * kept.  Workspace: la_gate_select_workspace bytes (pooled keys and the gate
+ * rows).  kbar (optional): the block means of k, (B, Hkv, n_kb, D)
  * fp64 contiguous as la_block_means writes them; given, k is not read and
  * not pooled (the per-step pooling of selection.py:620-624 is replaced by
  * means kept up to date on append).

@@ -115,48 +115,185 @@ __global__ __launch_bounds__(NT) void mean_pool_vec_kernel(const void *x, int dt
   }
 }
 
-constexpr int BS_DC = 32, BS_NT = 256;
+// scores[(b*Hq+h)*nq + i][j] = sum_d fl(q[b,h,i,d] * kbar[b,h/G,j,d]), fp64, d
+// increasing, each product rounded before it is added.  Row i sits at position
+// pos0 + i*qunit and column j starts at j*kunit: columns past every row of a
+// group are skipped (causal: their scores are never read).
+struct ScKP {
+  const void *q;  // at element strides q_sb, q_sh, q_st, unit stride over d
+  const double *kbar;
+  double *scores;
+  int64_t q_sb, q_sh, q_st;
+  int64_t Hq, Hkv, nq, nkb, D, pos0, qunit, kunit;
+  int32_t q_dt;
+};
 
-// scores[(b*Hq+h)*nqb + i][j] = sum_d fl(qbar[b,h,i,d] * kbar[b,h/G,j,d]) for
-// the TQ x TK tile (i, j), TK = (256 / (TQ / RQ)) * RK: each thread holds
-// RQ x RK scores.  Row i sits at position pos0 + i*qunit and column j starts
-// at j*kunit; tiles whose every column starts past every row's position are
-// skipped (causal: their scores are never read).  TQ = 64 (4 x 4 per thread)
-// for prefill rows; TQ = 4 (one score per thread, 64 columns) for decode,
-// where a 64-row tile would compute 63 empty rows per query.
-template <int TQ, int RQ, int RK>
-__global__ __launch_bounds__(BS_NT) void block_score_kernel(const double *qbar, const double *kbar,
-                                                            int64_t Hq, int64_t Hkv, int64_t nqb,
-                                                            int64_t nkb, int64_t D, int64_t pos0,
-                                                            int64_t qunit, int64_t kunit,
-                                                            double *scores) {
-  constexpr int TY = TQ / RQ, TX = BS_NT / TY, TK = TX * RK;
-  static_assert(TY * TX == BS_NT, "tile shape");
+constexpr int SC_NC = 8, SC_D = 128;  // columns of a wave, most dims
+
+template <int DT>
+__device__ __forceinline__ double sc_widen(const uint4 &v, int i) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  if constexpr (DT == LA_F32)
+    return (double)__uint_as_float(w[i]);
+  else if constexpr (DT == LA_BF16)
+    return (double)((i & 1) ? bf16hi(w[i / 2]) : bf16lo(w[i / 2]));
+  else
+    return (double)__half2float(__ushort_as_half((uint16_t)(w[i / 2] >> (16 * (i & 1)))));
+}
+
+// Many rows of q as stored (the gates): a lane is R rows; a workgroup takes 64 R
+// rows and 4 SC_NC columns, SC_NC per wave.  The columns' means sit in LDS and
+// are read as broadcasts; q is read in its own type, by the four waves together
+// (widened ahead of time it cost a pass of its own: 27 us for 1024 queries of 32
+// heads).  Bound by its fp64 instructions (a multiply and an add per product: they
+// round separately) and the broadcasts that feed them.  The scores leave through
+// LDS as runs of 4 SC_NC per row: written SC_NC at a time, at the power-of-two
+// strides that rows have, they took longer than the products.  1024 queries of 32
+// heads on 64 blocks, D = 128: 59 us with the widening pass and 4 x 4 scores per
+// thread, 27 like this.  Rows of 8-byte values (pooled q) need four times as many
+// scattered loads and stay with block_score_kernel (64 heads of 512 x 512, causal:
+// 208 us there, 205-290 in forms of this one).
+template <int DT, int R>
+__global__ __launch_bounds__(256) void row_score_kernel(ScKP p) {
+  constexpr int EV = DT == LA_F32 ? 4 : 8;  // values of a 16-byte load
+  constexpr int ESZ = 16 / EV, NL = 8 / EV;
+  constexpr int WC = 4 * SC_NC, LD = WC + 1, ROWS = 64 * R;
+  extern __shared__ __align__(16) double lds[];  // WC columns of D means; then ROWS rows of LD scores
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t j0 = (int64_t)blockIdx.x * WC, i0 = (int64_t)blockIdx.y * ROWS;
+  const int64_t bh = blockIdx.z, b = bh / p.Hq, h = bh % p.Hq;
+  // columns that start past every row's position: never read
+  const int64_t last = p.pos0 + min(i0 + ROWS - 1, p.nq - 1) * p.qunit;
+  if (j0 * p.kunit > last) return;
+  const int D = (int)p.D, nc = (int)min((int64_t)WC, p.nkb - j0);
+  const double *kr = p.kbar + ((b * p.Hkv + h / (p.Hq / p.Hkv)) * p.nkb + j0) * D;
+  for (int x = tid; x < WC * D; x += 256) lds[x] = x < nc * D ? kr[x] : 0.0;
+  __syncthreads();
+  double acc[R][SC_NC];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < SC_NC; ++c) acc[r][c] = 0.0;
+  if (SC_NC * w < nc && (j0 + SC_NC * w) * p.kunit <= last) {
+    const double *sk = lds + SC_NC * w * D;
+    const char *qr[R];
+    uint4 nx[R][NL];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      qr[r] = (const char *)p.q + (b * p.q_sb + h * p.q_sh + min(i0 + 64 * r + lane, p.nq - 1) * p.q_st) * ESZ;
+#pragma unroll
+      for (int y = 0; y < NL; ++y) nx[r][y] = *(const uint4 *)(qr[r] + 16 * y);
+    }
+    for (int d0 = 0; d0 < D; d0 += 8) {
+      double x[R][8];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[r][e] = sc_widen<DT>(nx[r][e / EV], e % EV);
+        if (d0 + 8 < D) {
+#pragma unroll
+          for (int y = 0; y < NL; ++y) nx[r][y] = *(const uint4 *)(qr[r] + (d0 + 8) * ESZ + 16 * y);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; e += 2)
+#pragma unroll
+        for (int c = 0; c < SC_NC; ++c) {
+          const double2 k2 = *(const double2 *)&sk[c * D + d0 + e];
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+            acc[r][c] = add_product(add_product(acc[r][c], x[r][e], k2.x), x[r][e + 1], k2.y);
+        }
+    }
+  }
+  __syncthreads();  // the means are read
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int c = 0; c < SC_NC; ++c) lds[(64 * r + lane) * LD + SC_NC * w + c] = acc[r][c];
+  __syncthreads();
+  const int nr = (int)min((int64_t)ROWS, p.nq - i0);
+  double *out = p.scores + (bh * p.nq + i0) * p.nkb + j0;
+  for (int x = tid; x < nr * WC; x += 256) {
+    const int i = x / WC, c = x % WC;
+    if (c < nc) out[i * p.nkb + c] = lds[i * LD + c];
+  }
+}
+
+// Few rows (decode): the heads of a KV head and their rows (at most SF_ROWS
+// together) against 64 columns; the columns' means, read once for all of
+// them, land in LDS in one memory round trip.  Bound by that read.
+constexpr int SF_ROWS = 8, SF_D = 128;
+__global__ __launch_bounds__(256) void few_row_score_kernel(ScKP p) {
+  __shared__ double sk[64][SF_D + 1];
+  __shared__ __align__(16) double sq[SF_ROWS][SF_D];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int64_t j0 = (int64_t)blockIdx.x * 64;
+  const int64_t kvh = blockIdx.y, b = blockIdx.z, G = p.Hq / p.Hkv;
+  if (j0 * p.kunit > p.pos0 + (p.nq - 1) * p.qunit) return;
+  const int D = (int)p.D, nc = (int)min((int64_t)64, p.nkb - j0), rows = (int)(G * p.nq);
+  const double *kr = p.kbar + ((b * p.Hkv + kvh) * p.nkb + j0) * D;
+  constexpr int PER = 64 * SF_D / 2 / 256;
+  const int total = nc * D / 2;
+  double2 v[PER];
+#pragma unroll
+  for (int x = 0; x < PER; ++x)
+    v[x] = tid + 256 * x < total ? ((const double2 *)kr)[tid + 256 * x] : double2{0.0, 0.0};
+  for (int x = tid; x < rows * D; x += 256) {
+    const int r = x / D, d = x % D;  // row r = (head g, row i)
+    sq[r][d] = load_as_f64(p.q, b * p.q_sb + (kvh * G + r / p.nq) * p.q_sh + (r % p.nq) * p.q_st + d, p.q_dt);
+  }
+#pragma unroll
+  for (int x = 0; x < PER; ++x) {
+    const int at = 2 * (tid + 256 * x);
+    if (at < 2 * total) {
+      sk[at / D][at % D] = v[x].x;
+      sk[at / D][at % D + 1] = v[x].y;
+    }
+  }
+  __syncthreads();
+  for (int r = w; r < rows; r += 4) {
+    double acc = 0.0;
+    for (int d = 0; d < D; ++d) acc = add_product(acc, sq[r][d], sk[lane][d]);
+    if (lane < nc)
+      p.scores[((b * p.Hq + kvh * G + r / p.nq) * p.nq + r % p.nq) * p.nkb + j0 + lane] = acc;
+  }
+}
+
+// Any shape (and pooled q, F64): 4 x 4 scores per thread on 64 x 64 tiles staged
+// in LDS.
+constexpr int BS_DC = 32, BS_NT = 256;
+template <bool F64>
+__global__ __launch_bounds__(BS_NT) void block_score_kernel(ScKP p) {
+  constexpr int TQ = 64, RQ = 4, RK = 4, TX = BS_NT / (TQ / RQ), TK = TX * RK;
   __shared__ double sq[BS_DC][TQ + 2];
   __shared__ double sk[BS_DC][TK + 2];
   const int tid = threadIdx.x;
   const int tq = tid / TX, tk = tid % TX;  // rows RQ*tq.., cols RK*tk..
   const int64_t i0 = (int64_t)blockIdx.y * TQ, j0 = (int64_t)blockIdx.x * TK;
   const int64_t bh = blockIdx.z;
-  const int64_t b = bh / Hq, h = bh % Hq;
-  if (j0 * kunit > pos0 + min(i0 + TQ - 1, nqb - 1) * qunit) return;  // all in the future
-  const double *qb = qbar + bh * nqb * D;
-  const double *kb = kbar + (b * Hkv + h / (Hq / Hkv)) * nkb * D;
+  const int64_t b = bh / p.Hq, h = bh % p.Hq;
+  if (j0 * p.kunit > p.pos0 + min(i0 + TQ - 1, p.nq - 1) * p.qunit) return;  // all in the future
+  const int64_t q0 = b * p.q_sb + h * p.q_sh;
+  const double *kb = p.kbar + (b * p.Hkv + h / (p.Hq / p.Hkv)) * p.nkb * p.D;
   double acc[RQ][RK];
 #pragma unroll
   for (int a = 0; a < RQ; ++a)
 #pragma unroll
     for (int c = 0; c < RK; ++c) acc[a][c] = 0.0;
-  for (int64_t d0 = 0; d0 < D; d0 += BS_DC) {
-    const int dn = (int)min((int64_t)BS_DC, D - d0);
+  for (int64_t d0 = 0; d0 < p.D; d0 += BS_DC) {
+    const int dn = (int)min((int64_t)BS_DC, p.D - d0);
     __syncthreads();
     for (int x = tid; x < TQ * BS_DC; x += BS_NT) {
       const int r = x / BS_DC, dd = x % BS_DC;
-      sq[dd][r] = (dd < dn && i0 + r < nqb) ? qb[(i0 + r) * D + d0 + dd] : 0.0;
+      const int64_t at = q0 + (i0 + r) * p.q_st + d0 + dd;
+      double v = 0.0;
+      if (dd < dn && i0 + r < p.nq) v = F64 ? ((const double *)p.q)[at] : load_as_f64(p.q, at, p.q_dt);
+      sq[dd][r] = v;
     }
     for (int x = tid; x < TK * BS_DC; x += BS_NT) {
       const int r = x / BS_DC, dd = x % BS_DC;
-      sk[dd][r] = (dd < dn && j0 + r < nkb) ? kb[(j0 + r) * D + d0 + dd] : 0.0;
+      sk[dd][r] = (dd < dn && j0 + r < p.nkb) ? kb[(j0 + r) * p.D + d0 + dd] : 0.0;
     }
     __syncthreads();
     for (int dd = 0; dd < dn; ++dd) {
@@ -174,30 +311,48 @@ __global__ __launch_bounds__(BS_NT) void block_score_kernel(const double *qbar, 
 #pragma unroll
   for (int a = 0; a < RQ; ++a) {
     const int64_t i = i0 + RQ * tq + a;
-    if (i >= nqb) continue;
+    if (i >= p.nq) continue;
 #pragma unroll
     for (int c = 0; c < RK; ++c) {
       const int64_t j = j0 + RK * tk + c;
-      if (j < nkb) scores[(bh * nqb + i) * nkb + j] = acc[a][c];
+      if (j < p.nkb) p.scores[(bh * p.nq + i) * p.nkb + j] = acc[a][c];
     }
   }
 }
 
-// Scores of every (row, column) tile of (B * Hq) heads; the tile shape
-// follows the number of rows.
-static void block_scores(const double *qbar, const double *kbar, int64_t B, int64_t Hq,
-                         int64_t Hkv, int64_t nqb, int64_t nkb, int64_t D, int64_t pos0,
-                         int64_t qunit, int64_t kunit, double *scores, hipStream_t st) {
-  if (nqb <= 4)
-    block_score_kernel<4, 1, 1><<<dim3((unsigned)ceil_div(nkb, 64), (unsigned)ceil_div(nqb, 4),
-                                       (unsigned)(B * Hq)),
-                                  BS_NT, 0, st>>>(qbar, kbar, Hq, Hkv, nqb, nkb, D, pos0, qunit,
-                                                  kunit, scores);
+template <int DT>
+static void launch_row_scores(const ScKP &p, int64_t B, hipStream_t st) {
+  const int R = p.nq > 64 ? 2 : 1;
+  const dim3 grid((unsigned)ceil_div(p.nkb, 4 * SC_NC), (unsigned)ceil_div(p.nq, 64 * R), (unsigned)(B * p.Hq));
+  const size_t lds = std::max<size_t>(4 * SC_NC * p.D, 64 * R * (4 * SC_NC + 1)) * sizeof(double);
+  if (R == 2)
+    row_score_kernel<DT, 2><<<grid, 256, lds, st>>>(p);
   else
-    block_score_kernel<64, 4, 4><<<dim3((unsigned)ceil_div(nkb, 64), (unsigned)ceil_div(nqb, 64),
-                                        (unsigned)(B * Hq)),
-                                   BS_NT, 0, st>>>(qbar, kbar, Hq, Hkv, nqb, nkb, D, pos0, qunit,
-                                                   kunit, scores);
+    row_score_kernel<DT, 1><<<grid, 256, lds, st>>>(p);
+}
+
+// Scores of every row and column of (B * Hq) heads.  Up to SF_ROWS rows per KV
+// head take the decode form; the row form needs q rows in 16-byte pieces, and
+// below 16 rows its lanes are mostly idle.
+static void block_scores(const ScKP &p, int64_t B, hipStream_t st) {
+  const int64_t ev = p.q_dt == LA_F32 ? 4 : 8;
+  if (p.Hq / p.Hkv * p.nq <= SF_ROWS && p.D <= SF_D && p.D % 2 == 0 && (uintptr_t)p.kbar % 16 == 0) {
+    few_row_score_kernel<<<dim3((unsigned)ceil_div(p.nkb, 64), (unsigned)p.Hkv, (unsigned)B), 256, 0, st>>>(p);
+    return;
+  }
+  const dim3 tiles((unsigned)ceil_div(p.nkb, 64), (unsigned)ceil_div(p.nq, 64), (unsigned)(B * p.Hq));
+  const bool rows = p.nq >= 16 && p.D % 8 == 0 && p.D <= SC_D && (uintptr_t)p.q % 16 == 0 &&
+                    p.q_sb % ev == 0 && p.q_sh % ev == 0 && p.q_st % ev == 0;
+  if (p.q_dt == LA_F64)
+    block_score_kernel<true><<<tiles, BS_NT, 0, st>>>(p);
+  else if (!rows)
+    block_score_kernel<false><<<tiles, BS_NT, 0, st>>>(p);
+  else if (p.q_dt == LA_F32)
+    launch_row_scores<LA_F32>(p, B, st);
+  else if (p.q_dt == LA_BF16)
+    launch_row_scores<LA_BF16>(p, B, st);
+  else
+    launch_row_scores<LA_F16>(p, B, st);
 }
 
 // Mean of every `bs` rows of x[b][h] (rows past T_b repeat row T_b-1) into
@@ -283,7 +438,21 @@ extern "C" int la_block_select(const la_block_select_args *a, void *stream) {
   pool_rows(a->k, a->in_dtype, a->B, a->Hkv, a->T, a->D, a->k_sb, a->k_sh, a->k_st, a->block, L.nkb,
             kbar, st, a->lengths);
   LA_LAUNCHED();
-  block_scores(qbar, kbar, a->B, a->Hq, a->Hkv, L.nqb, L.nkb, a->D, 0, 1, 1, sc, st);
+  ScKP sp{};
+  sp.q = qbar;
+  sp.q_dt = LA_F64;
+  sp.q_st = a->D;
+  sp.q_sh = L.nqb * a->D;
+  sp.q_sb = a->Hq * L.nqb * a->D;
+  sp.kbar = kbar;
+  sp.scores = sc;
+  sp.Hq = a->Hq;
+  sp.Hkv = a->Hkv;
+  sp.nq = L.nqb;
+  sp.nkb = L.nkb;
+  sp.D = a->D;
+  sp.qunit = sp.kunit = 1;
+  block_scores(sp, a->B, st);
   LA_LAUNCHED();
   TopkKParams tp{};
   tp.scores = sc;
@@ -320,13 +489,12 @@ extern "C" int la_block_select(const la_block_select_args *a, void *stream) {
 // the ranking); ties go to the lowest block.
 namespace la {
 struct GsLayout {
-  int64_t nkb, qbar_off, kbar_off, sc_off, bytes;
+  int64_t nkb, kbar_off, sc_off, bytes;
 };
 static GsLayout gs_layout(const la_gate_select_args *a) {
   GsLayout L{};
   L.nkb = ceil_div(a->T, a->block);
-  L.qbar_off = 0;
-  L.kbar_off = L.qbar_off + a->B * a->Hq * a->Tq * a->D * 8;
+  L.kbar_off = 0;
   // (no pooled keys when the caller keeps them)
   L.sc_off = L.kbar_off + (a->kbar ? 0 : a->B * a->Hkv * L.nkb * a->D * 8);
   L.bytes = L.sc_off + a->B * a->Hq * a->Tq * L.nkb * 8;
@@ -362,12 +530,8 @@ extern "C" int la_gate_select(const la_gate_select_args *a, void *stream) {
                 (long long)a->ws_bytes, (long long)L.bytes);
   hipStream_t st = (hipStream_t)stream;
   char *ws = (char *)a->workspace;
-  double *qbar = (double *)(ws + L.qbar_off);
   double *kbar = (double *)(ws + L.kbar_off);
   double *sc = (double *)(ws + L.sc_off);
-  pool_rows(a->q, a->in_dtype, a->B, a->Hq, a->Tq, a->D, a->q_sb, a->q_sh, a->q_st, 1, a->Tq, qbar,
-            st);  // q widened to fp64
-  LA_LAUNCHED();
   if (a->kbar) {  // block means kept by the caller (la_block_means)
     kbar = const_cast<double *>(a->kbar);
   } else {
@@ -375,8 +539,23 @@ extern "C" int la_gate_select(const la_gate_select_args *a, void *stream) {
               L.nkb, kbar, st);
     LA_LAUNCHED();
   }
-  block_scores(qbar, kbar, a->B, a->Hq, a->Hkv, a->Tq, L.nkb, a->D, a->offset, 1, a->block, sc,
-               st);
+  ScKP sp{};
+  sp.q = a->q;
+  sp.q_dt = a->in_dtype;
+  sp.q_sb = a->q_sb;
+  sp.q_sh = a->q_sh;
+  sp.q_st = a->q_st;
+  sp.kbar = kbar;
+  sp.scores = sc;
+  sp.Hq = a->Hq;
+  sp.Hkv = a->Hkv;
+  sp.nq = a->Tq;
+  sp.nkb = L.nkb;
+  sp.D = a->D;
+  sp.pos0 = a->offset;
+  sp.qunit = 1;
+  sp.kunit = a->block;
+  block_scores(sp, a->B, st);
   LA_LAUNCHED();
   TopkKParams tp{};
   tp.scores = sc;

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define LA_ABI_VERSION 13
+#define LA_ABI_VERSION 14
 
 /* element types */
 enum {
@@ -181,6 +181,20 @@ int la_sparse_attention(const la_sparse_attn_args *a, const la_kv *kv, void *str
  */
 #define LA_NOALLOC_MAX_WORKSPACE ((size_t)16 << 20)
 int la_sparse_attention_noalloc(const la_sparse_attn_args *a, const la_kv *kv, void *stream);
+
+/*
+ * Totals of list reads, for read accounting (core.py:281-306 reports means of
+ * them): totals[0] = the tokens the lists cover, entry u of a row at position
+ * offset + t covering the tokens of [u*unit, (u+1)*unit) below
+ * min(offset + t + 1, t_k) (-1 entries none); totals[1] = the sum of `counts`
+ * (n_counts of them; NULL: 0).  ids: [B][L][ceil(Tq/rep)][W] at element strides
+ * id_sb/id_sh/id_st (0 allowed), each list shared by `rep` consecutive
+ * queries.  totals: two device words, written (not added to).
+ */
+int la_list_reads(const int32_t *ids, int64_t id_sb, int64_t id_sh, int64_t id_st, int64_t B,
+                  int64_t L, int64_t Tq, int64_t W, int64_t rep, int64_t unit, int64_t offset,
+                  int64_t t_k, const int32_t *counts, int64_t n_counts, uint64_t *totals,
+                  void *stream);
 
 /*
  * Quest page metadata: channel-wise min / max of the keys of every page.

@@ -16,7 +16,7 @@ from typing import Optional
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "liblinattn_hip.so"
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 LA_F32, LA_BF16, LA_F16, LA_FP8_E4M3, LA_F64 = 0, 1, 2, 3, 4
 LA_OK, LA_ERR_INVALID, LA_ERR_UNSUPPORTED, LA_ERR_HIP, LA_ERR_WORKSPACE = 0, 1, 2, 3, 4
@@ -27,6 +27,7 @@ EXPORTED = (
     "la_sparse_attention_workspace",
     "la_sparse_attention",
     "la_sparse_attention_noalloc",
+    "la_list_reads",
     "la_quest_page_bounds",
     "la_quest_scores",
     "la_quest_select",
@@ -189,6 +190,7 @@ def load() -> ctypes.CDLL:
     L.la_sparse_attention_workspace.restype = ctypes.c_size_t
     L.la_sparse_attention.argtypes = [P(LaSparseAttnArgs), P(LaKV), _vp]
     L.la_sparse_attention_noalloc.argtypes = [P(LaSparseAttnArgs), P(LaKV), _vp]
+    L.la_list_reads.argtypes = [_vp] + [_i64] * 11 + [_vp, _i64, _vp, _vp]
     L.la_quest_page_bounds.argtypes = [P(LaKV), _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp,
                                        _i64, _i64, _i64, _i64, _i32, _vp]
     L.la_quest_scores.argtypes = [_vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp,

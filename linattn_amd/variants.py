@@ -28,6 +28,7 @@ from typing import Any, Dict, Optional
 
 import torch
 
+from linattn_amd import _native as N
 from linattn_amd.core import AttnConfig, AttentionVariant
 from linattn_amd.kernels.block_sparse import sparse_attention
 from linattn_amd.kernels.fused_indexer import indexer_topk
@@ -39,15 +40,43 @@ __all__ = ["HipAttention", "HipQuest", "HipDSA", "HipMoBA", "HipXAttention", "Hi
            "HipStreamingSink", "SUPPORTED"]
 
 
-def _reads_per_query(ids: torch.Tensor, unit: int, offset: int, t_k: int) -> float:
-    """Mean tokens read per query row: listed units intersected with
-    causality and the cache length (ids (B, L, Tq, W), -1 padded)."""
-    tq = ids.shape[2]
-    lim = torch.clamp(torch.arange(tq, device=ids.device) + offset + 1, max=t_k)
-    start = ids.to(torch.int64) * unit
-    n = torch.clamp(lim.view(1, 1, tq, 1) - start, min=0, max=unit)
-    n = torch.where(ids >= 0, n, torch.zeros_like(n))
-    return float(n.sum(-1).to(torch.float64).mean())
+class _Totals:
+    """Token reads and counts of one selection, summed on the device
+    (``la_list_reads``) with no host read until a mean is asked for."""
+
+    def __init__(self, ids: torch.Tensor, unit: int, offset: int, t_q: int, t_k: int,
+                 counts: Optional[torch.Tensor] = None, rep: int = 1):
+        """ids (B, L, rows, W), -1 padded: rows = ceil(t_q / rep), or 1 list
+        shared by every query; listed units are intersected with causality and
+        the cache length."""
+        B, L, rows, W = ids.shape
+        sb, sh, st = ids.stride(0), ids.stride(1), ids.stride(2)
+        if ids.stride(3) != 1:
+            ids = ids.contiguous()
+            sb, sh, st = ids.stride(0), ids.stride(1), ids.stride(2)
+        self.totals = torch.empty(2, dtype=torch.int64, device=ids.device)
+        self.stream = torch.cuda.current_stream(ids.device)
+        self.rows = B * L * t_q
+        self.lists = counts.numel() if counts is not None else 0
+        self._host = None
+        N.check(N.load().la_list_reads(
+            ids.data_ptr(), sb, sh, 0 if rows == 1 else st, B, L, t_q, W, rep, unit, offset, t_k,
+            N.ptr(counts), self.lists, self.totals.data_ptr(), self.stream.cuda_stream),
+            "read totals")
+
+    def _read(self):
+        if self._host is None:
+            self.stream.synchronize()
+            self._host = self.totals.tolist()
+        return self._host
+
+    def reads(self) -> float:
+        """Mean tokens read per query row."""
+        return self._read()[0] / self.rows
+
+    def counts(self) -> float:
+        """Mean entries per list."""
+        return self._read()[1] / self.lists
 
 
 class HipAttention(AttentionVariant):
@@ -59,10 +88,10 @@ class HipAttention(AttentionVariant):
     def __init__(self, cfg: Optional[AttnConfig] = None, **kw: Any):
         super().__init__(cfg, **kw)
         self.name = f"hip_{self.reference}"
-        self._extra: Dict[str, float] = {}
+        self._extra: Dict[str, Any] = {}  # floats, or what reads one off the device
 
     def stats(self) -> Dict[str, float]:
-        return dict(self._extra)
+        return {k: v() if callable(v) else v for k, v in self._extra.items()}
 
     def forward(self, q, k, v, *, state=None, chunk=None, causal=True, collect_stats=False):
         """The reference driver (core.py:231-279).  fp64 inputs (the reference
@@ -131,12 +160,13 @@ class HipQuest(HipAttention):
             ids, counts = quest_select_hip(q, state["page_min"], state["page_max"], page_size=ps,
                                            topk=self.cfg.topk_blocks, offset=offset,
                                            gqa_union=self.gqa_union)
-            self._extra = {"pages_per_query": float(counts.to(torch.float64).mean())}
+            self._extra = {}
         out = sparse_attention(q, k, v, ids, unit=ps, counts=counts, causal=True, offset=offset,
                                out_dtype=q.dtype)
-        reads = _reads_per_query(ids if ids.shape[2] == q.shape[2] else
-                                 ids.expand(-1, -1, q.shape[2], -1), ps, offset, t_k)
-        self._extra["reads_per_query"] = reads
+        tot = _Totals(ids, ps, offset, q.shape[2], t_k, counts)
+        if counts is not None:
+            self._extra["pages_per_query"] = tot.counts
+        self._extra["reads_per_query"] = tot.reads
         return out
 
     def read_budget(self, seq_len, batch=1):
@@ -170,7 +200,7 @@ class HipSlidingWindow(HipAttention):
         ids = lists.view(1, 1, q.shape[2], -1).expand(q.shape[0], k.shape[1], -1, -1)
         out = sparse_attention(q, k, v, ids, unit=1, causal=True, offset=offset,
                                out_dtype=q.dtype)
-        self._extra = {"reads_per_query": _reads_per_query(ids, 1, offset, k.shape[-2])}
+        self._extra = {"reads_per_query": _Totals(ids, 1, offset, q.shape[2], k.shape[-2]).reads}
         return out
 
     def read_budget(self, seq_len, batch=1):
@@ -287,7 +317,7 @@ class HipDSA(HipAttention):
         ids = self.select_lists(q, k, offset)
         out = sparse_attention(q, k, v, ids, unit=1, causal=True, offset=offset,
                                out_dtype=q.dtype)
-        reads = _reads_per_query(ids, 1, offset, k.shape[-2])
+        reads = _Totals(ids, 1, offset, q.shape[2], k.shape[-2]).reads
         self._extra = {"reads_per_query": reads, "tokens_per_query": reads}
         return out
 
@@ -347,8 +377,8 @@ class HipMoBA(HipAttention):
                                       kbar=state.get("block_means"))
         out = sparse_attention(q, k, v, ids, unit=bs, counts=counts, causal=True, offset=offset,
                                out_dtype=q.dtype)
-        self._extra = {"blocks_per_query": float(counts.to(torch.float64).mean()),
-                       "reads_per_query": _reads_per_query(ids, bs, offset, k.shape[-2])}
+        tot = _Totals(ids, bs, offset, q.shape[2], k.shape[-2], counts)
+        self._extra = {"blocks_per_query": tot.counts, "reads_per_query": tot.reads}
         return out
 
     def read_budget(self, seq_len, batch=1):
@@ -408,14 +438,13 @@ class HipXAttention(HipAttention):
         if (blk == 64 and offset == 0 and Tq == T and q.shape[3] == 128
                 and q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16):
             out = block_sparse_prefill(q, k, v, ids, counts, block_size=64, out_dtype=q.dtype)
-            rows = ids.repeat_interleave(blk, dim=2)[:, :, :Tq]
         else:
             rows = ids.repeat_interleave(blk, dim=2)[:, :, :Tq].contiguous()
             rcounts = counts.repeat_interleave(blk, dim=2)[:, :, :Tq].contiguous()
             out = sparse_attention(q, k, v, rows, unit=blk, counts=rcounts, causal=True,
                                    offset=offset, out_dtype=q.dtype)
-        self._extra = {"blocks_per_query": float(counts.to(torch.float64).mean()),
-                       "reads_per_query": _reads_per_query(rows, blk, offset, T)}
+        tot = _Totals(ids, blk, offset, Tq, T, counts, rep=blk)
+        self._extra = {"blocks_per_query": tot.counts, "reads_per_query": tot.reads}
         return out
 
     def read_budget(self, seq_len, batch=1):

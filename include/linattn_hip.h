@@ -263,6 +263,17 @@ typedef struct {
 int la_quest_select(const la_quest_select_args *a, void *stream);
 
 /*
+ * The same selection per query head, without the union (selection.py:214-231,
+ * gqa_union off): out_idx[((b*Hq + h)*Tq + t)*k + i] holds the head's pages by
+ * (score desc, index asc), -1 padded, out_count the number kept.  Identical to
+ * la_quest_scores followed by la_topk_rows with group = 1, order = 0, force_own =
+ * 1, pos_unit = page_size.  Returns LA_ERR_UNSUPPORTED (nothing launched) when
+ * the metadata is not page-minor (m_sp == 1), for more than 1024 pages or for
+ * k > 256; callers then use the two separate entry points.
+ */
+int la_quest_select_heads(const la_quest_select_args *a, void *stream);
+
+/*
  * Fused Quest decode: page selection and attention in one kernel, the
  * fusion of selector and decode kernel that docs/kernels.md:89-93 describes
  * (FFD) beyond the fused top-k of quest_pages.py:110-113: the selected page

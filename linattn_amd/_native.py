@@ -31,6 +31,7 @@ EXPORTED = (
     "la_quest_page_bounds",
     "la_quest_scores",
     "la_quest_select",
+    "la_quest_select_heads",
     "la_quest_decode_fused",
     "la_topk_rows_workspace",
     "la_topk_rows",
@@ -196,6 +197,7 @@ def load() -> ctypes.CDLL:
     L.la_quest_scores.argtypes = [_vp, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp,
                                   _i32, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp]
     L.la_quest_select.argtypes = [P(LaQuestSelectArgs), _vp]
+    L.la_quest_select_heads.argtypes = [P(LaQuestSelectArgs), _vp]
     L.la_quest_decode_fused.argtypes = [P(LaQuestDecodeArgs), _vp]
     L.la_topk_rows_workspace.argtypes = [P(LaTopkArgs)]
     L.la_topk_rows_workspace.restype = ctypes.c_size_t

@@ -298,6 +298,133 @@ __global__ __launch_bounds__(qs_nt<KPT>()) void quest_select_kernel(QsKP a) {
                             a.out_count ? a.out_count + row : nullptr, wtmp);
 }
 
+// Per-head selection of one (b, query head, query t) row, by score: the page
+// scores (as in quest_scores_kernel), the own page forced, the top k in (score
+// desc, index asc) order, equal to quest_scores_kernel and the sorted top-k.
+// A lane takes pages lane + 64 j; q_d is wave-uniform, so its sign picks the one
+// bound a page contributes (half the metadata is read) and its value is a scalar
+// operand.  Short rows are latency chains, so the row's scores, selection and
+// ranking are one kernel: NWR waves score a row (four when rows are few), one
+// selects it, ranking the kept pages against each other in LDS.  8 rows of 256
+// pages, D = 64: 20 us in two launches, 13 us here; 2048 rows of at most 32: 39
+// us and 15.
+template <int MT, int KPL, int NWR>
+__global__ __launch_bounds__(256) void quest_head_select_kernel(QsKP a, int64_t rows) {
+  constexpr int NP = 64 * KPL, RPW = 4 / NWR, SL = KPL / NWR;
+  static_assert(KPL % NWR == 0, "slots of a scoring wave");
+  __shared__ uint64_t keys[RPW][NP];
+  __shared__ uint16_t sidx[RPW][NP];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rl = w / NWR, part = w % NWR;
+  const int64_t row = (int64_t)blockIdx.x * RPW + rl;  // (b, h, t)
+  const bool live = row < rows;
+  const uint32_t r32 = (uint32_t)(live ? row : rows - 1);
+  const uint32_t bh = r32 / (uint32_t)a.Tq, t = r32 - bh * (uint32_t)a.Tq;
+  const uint32_t b = bh / (uint32_t)a.Hq, h = bh - b * (uint32_t)a.Hq;
+  const int64_t pos = (a.positions ? (int64_t)a.positions[b] : a.pos_offset) + t;
+  const int64_t u_own = pos < 0 ? -1
+                        : pos < ((int64_t)1 << 32) && a.page_size < ((int64_t)1 << 32)
+                            ? (int64_t)((uint32_t)pos / (uint32_t)a.page_size)
+                            : pos / a.page_size;
+  const int32_t n_v = (int32_t)min(a.n_pages, u_own + 1);
+  const int32_t own = (int32_t)min(u_own, a.n_pages - 1);
+  const bool force = own >= 0 && own < n_v;
+  const int D = (int)a.D;
+  const int64_t qo = b * a.q_sb + h * a.q_sh + (int64_t)t * a.q_st;
+  const int64_t mbase = b * a.m_sb + (h / (uint32_t)(a.Hq / a.Hkv)) * a.m_sh;
+  double acc[SL];
+  int64_t pg[SL];  // pages past the end re-read the last one (not consumed)
+#pragma unroll
+  for (int j = 0; j < SL; ++j) {
+    acc[j] = 0.0;
+    pg[j] = mbase + min((int64_t)(lane + 64 * (part * SL + j)), a.n_pages - 1);
+  }
+  if (64 * part * SL < n_v) {  // (wave-uniform)
+    using E = typename std::conditional<MT == LA_BF16, uint16_t, float>::type;
+    for (int c = 0; c < D; c += 64) {
+      const double qv = c + lane < D ? load_as_f64(a.q, qo + c + lane, a.q_dt) : 0.0;
+      const uint64_t qbits = (uint64_t)__double_as_longlong(qv);
+      const int dn = min(64, D - c);
+      constexpr int QD = SL == 1 ? 32 : SL == 2 ? 16 : 8;
+      for (int d0 = 0; d0 < dn; d0 += QD) {
+        E v[QD][SL];
+#pragma unroll
+        for (int e = 0; e < QD; ++e) {
+          const int d = min(d0 + e, dn - 1);
+          const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)qbits, d);
+          const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(qbits >> 32), d);
+          const uint32_t mag = hi & 0x7fffffffu;  // q < 0: the lower bound counts
+          const bool neg = (hi >> 31) && (mag | lo) != 0 && mag <= 0x7ff00000u;
+          const E *base = (const E *)(neg ? a.mn : a.mx) + (c + d) * a.m_sd;
+#pragma unroll
+          for (int j = 0; j < SL; ++j) v[e][j] = base[pg[j]];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every load is on its way
+#pragma unroll
+        for (int e = 0; e < QD; ++e) {
+          if (d0 + e >= dn) continue;
+          const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)qbits, d0 + e);
+          const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(qbits >> 32), d0 + e);
+          const double qd = __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+#pragma unroll
+          for (int j = 0; j < SL; ++j) {
+            double x;
+            if constexpr (MT == LA_BF16)
+              x = (double)bf16_bits_to_f32(v[e][j]);
+            else
+              x = (double)v[e][j];
+            acc[j] = __builtin_fma(qd, x, acc[j]);
+          }
+        }
+      }
+    }
+  }
+  uint64_t u[KPL];
+  if constexpr (NWR == 1) {
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) u[j] = (force && lane + 64 * j == own) ? KEY_FORCED : ord_key(acc[j]);
+    if (!live) return;  // (whole waves; no barrier follows)
+  } else {
+#pragma unroll
+    for (int j = 0; j < SL; ++j) {
+      const int i = lane + 64 * (part * SL + j);
+      keys[rl][i] = (force && i == own) ? KEY_FORCED : ord_key(acc[j]);
+    }
+    __syncthreads();
+    if (part != 0 || !live) return;
+#pragma unroll
+    for (int j = 0; j < KPL; ++j) u[j] = keys[rl][lane + 64 * j];
+    __builtin_amdgcn_wave_barrier();
+  }
+  // the kept pages in index order, then each to its rank
+  const int32_t K = (int32_t)min(a.k, (int64_t)n_v);
+  const uint64_t lt = lanemask_lt(lane);
+  int32_t at = 0;
+  tk_wave_select_bits<KPL>(u, n_v, (uint32_t)K, [&](int j, int32_t i, bool take) {
+    const uint64_t m = __ballot(take);
+    if (take) {
+      const int32_t x = at + (int32_t)__popcll(m & lt);
+      keys[rl][x] = u[j];
+      sidx[rl][x] = (uint16_t)i;
+    }
+    at += (int32_t)__popcll(m);
+  });
+  __builtin_amdgcn_wave_barrier();
+  int32_t *out = a.out_idx + row * a.width;
+  for (int32_t x0 = 0; x0 < K; x0 += 64) {
+    const int32_t x = x0 + lane;
+    const uint64_t mine = x < K ? keys[rl][x] : 0ull;
+    int32_t rank = 0;
+    for (int32_t y = 0; y < K; ++y) {
+      const uint64_t ky = keys[rl][y];
+      rank += (ky > mine || (ky == mine && y < x)) ? 1 : 0;
+    }
+    if (x < K) out[rank] = (int32_t)sidx[rl][x];
+  }
+  for (int64_t x = K + lane; x < a.width; x += 64) out[x] = -1;
+  if (a.out_count && lane == 0) a.out_count[row] = K;
+}
+
 template <int MT, int G>
 static int launch_scores(const void *q, int q_dt, int64_t B, int64_t Hq, int64_t Tq, int64_t D,
                          int64_t q_sb, int64_t q_sh, int64_t q_st, const void *mn, const void *mx,
@@ -436,7 +563,7 @@ static int launch_select_kpt(const QsKP &k, int64_t rows, hipStream_t st) {
   return fail(LA_ERR_UNSUPPORTED, "la_quest_select: too many pages for one workgroup");
 }
 
-extern "C" int la_quest_select(const la_quest_select_args *a, void *stream) {
+static int validate_select(const la_quest_select_args *a) {
   LA_REQUIRE(a && a->q && a->page_min && a->page_max && a->out_idx, "la_quest_select: null pointer");
   LA_REQUIRE(a->B > 0 && a->Hq > 0 && a->Tq > 0 && a->Hkv > 0 && a->n_pages > 0 && a->k > 0,
              "la_quest_select: bad shape");
@@ -446,14 +573,10 @@ extern "C" int la_quest_select(const la_quest_select_args *a, void *stream) {
   LA_REQUIRE(a->q_dtype == LA_F32 || a->q_dtype == LA_BF16 || a->q_dtype == LA_F16,
              "la_quest_select: q dtype");
   LA_REQUIRE(a->meta_dtype == LA_F32 || a->meta_dtype == LA_BF16, "la_quest_select: meta dtype");
-  const int64_t G = a->Hq / a->Hkv;
-  const int64_t esz = a->meta_dtype == LA_BF16 ? 2 : 4;
-  // page-minor metadata, 4 pages per aligned vector
-  const bool layout = a->m_sp == 1 && a->m_sd % 4 == 0 && a->m_sd >= a->n_pages &&
-                      a->m_sb % 4 == 0 && a->m_sh % 4 == 0 &&
-                      (uintptr_t)a->page_min % (4 * esz) == 0 && (uintptr_t)a->page_max % (4 * esz) == 0;
-  if (!layout || a->n_pages > (G <= 4 ? 4096 : 2048) || !(G == 1 || G == 2 || G == 4 || G == 8))
-    return fail(LA_ERR_UNSUPPORTED, "la_quest_select: shape or metadata layout not fused");
+  return LA_OK;
+}
+
+static QsKP select_params(const la_quest_select_args *a) {
   QsKP k{};
   k.q = a->q;
   k.mn = a->page_min;
@@ -475,8 +598,61 @@ extern "C" int la_quest_select(const la_quest_select_args *a, void *stream) {
   k.pos_offset = a->pos_offset;
   k.positions = a->positions;
   k.k = std::max<int64_t>(1, std::min(a->k, a->n_pages));
-  k.width = G * k.k;
   k.q_dt = a->q_dtype;
+  return k;
+}
+
+template <int MT>
+static int launch_head_select(const QsKP &k, int64_t rows, hipStream_t st) {
+  // four waves score a row while the rows leave SIMDs idle, one each above that
+  // (2048 rows fill the device's 1024 SIMDs twice)
+  const bool few = rows < 2048;
+  const dim3 one((unsigned)ceil_div(rows, 4)), four((unsigned)rows);
+  if (k.n_pages <= 64)
+    quest_head_select_kernel<MT, 1, 1><<<one, 256, 0, st>>>(k, rows);
+  else if (k.n_pages <= 128)
+    quest_head_select_kernel<MT, 2, 1><<<one, 256, 0, st>>>(k, rows);
+  else if (k.n_pages <= 256 && few)
+    quest_head_select_kernel<MT, 4, 4><<<four, 256, 0, st>>>(k, rows);
+  else if (k.n_pages <= 256)
+    quest_head_select_kernel<MT, 4, 1><<<one, 256, 0, st>>>(k, rows);
+  else if (k.n_pages <= 512)
+    quest_head_select_kernel<MT, 8, 4><<<four, 256, 0, st>>>(k, rows);
+  else
+    quest_head_select_kernel<MT, 16, 4><<<four, 256, 0, st>>>(k, rows);
+  LA_LAUNCHED();
+  return LA_OK;
+}
+
+extern "C" int la_quest_select_heads(const la_quest_select_args *a, void *stream) {
+  const int rc = validate_select(a);
+  if (rc != LA_OK) return rc;
+  const int64_t rows = a->B * a->Hq * a->Tq;
+  // page-minor metadata (any alignment); rows that one workgroup's LDS holds
+  const int64_t G = a->Hq / a->Hkv;
+  if (a->m_sp != 1 || a->n_pages > 1024 || rows >= ((int64_t)1 << 31) || std::min(a->k, a->n_pages) > 256 ||
+      !(G == 1 || G == 2 || G == 4 || G == 8))
+    return fail(LA_ERR_UNSUPPORTED, "la_quest_select_heads: shape or metadata layout not fused");
+  QsKP k = select_params(a);
+  k.width = k.k;
+  hipStream_t st = (hipStream_t)stream;
+  return a->meta_dtype == LA_BF16 ? launch_head_select<LA_BF16>(k, rows, st)
+                                  : launch_head_select<LA_F32>(k, rows, st);
+}
+
+extern "C" int la_quest_select(const la_quest_select_args *a, void *stream) {
+  const int rc = validate_select(a);
+  if (rc != LA_OK) return rc;
+  const int64_t G = a->Hq / a->Hkv;
+  const int64_t esz = a->meta_dtype == LA_BF16 ? 2 : 4;
+  // page-minor metadata, 4 pages per aligned vector
+  const bool layout = a->m_sp == 1 && a->m_sd % 4 == 0 && a->m_sd >= a->n_pages &&
+                      a->m_sb % 4 == 0 && a->m_sh % 4 == 0 &&
+                      (uintptr_t)a->page_min % (4 * esz) == 0 && (uintptr_t)a->page_max % (4 * esz) == 0;
+  if (!layout || a->n_pages > (G <= 4 ? 4096 : 2048) || !(G == 1 || G == 2 || G == 4 || G == 8))
+    return fail(LA_ERR_UNSUPPORTED, "la_quest_select: shape or metadata layout not fused");
+  QsKP k = select_params(a);
+  k.width = G * k.k;
   const int64_t rows = a->B * a->Hkv * a->Tq;
   hipStream_t st = (hipStream_t)stream;
 #define LA_QSEL(MT)                                                  \

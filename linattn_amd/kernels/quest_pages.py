@@ -163,10 +163,12 @@ def quest_select_hip(q: torch.Tensor, mins: torch.Tensor, maxs: torch.Tensor, *,
     if positions is not None and (positions.dtype != torch.int32 or positions.shape != (B,)
                                   or not positions.is_contiguous()):
         raise ValueError("positions must be contiguous int32 (B,)")
-    if gqa_union and G > 1 and mins.stride() == maxs.stride() and mins.dtype == maxs.dtype:
-        # one pass: scores, per-head top-k and the union (la_quest_select)
-        ids = torch.empty(B, Hkv, Tq, G * k, dtype=torch.int32, device=dev)
-        counts = torch.empty(B, Hkv, Tq, dtype=torch.int32, device=dev)
+    if mins.stride() == maxs.stride() and mins.dtype == maxs.dtype:
+        # one pass: scores and top-k per head, and the union of a group's heads
+        union = gqa_union and G > 1
+        heads, width = (Hkv, G * k) if union else (Hq, k)
+        ids = torch.empty(B, heads, Tq, width, dtype=torch.int32, device=dev)
+        counts = torch.empty(B, heads, Tq, dtype=torch.int32, device=dev)
         a = N.LaQuestSelectArgs()
         a.q, a.page_min, a.page_max = q.data_ptr(), mins.data_ptr(), maxs.data_ptr()
         a.out_idx, a.out_count = ids.data_ptr(), counts.data_ptr()
@@ -177,7 +179,9 @@ def quest_select_hip(q: torch.Tensor, mins: torch.Tensor, maxs: torch.Tensor, *,
         a.page_size, a.pos_offset, a.k = page_size, offset, k
         a.q_dtype, a.meta_dtype = N.dtype_code(q.dtype), N.dtype_code(mins.dtype)
         a.positions = N.ptr(positions)
-        rc = N.load().la_quest_select(ctypes.byref(a), N.stream_handle(dev))
+        L = N.load()
+        select = L.la_quest_select if union else L.la_quest_select_heads
+        rc = select(ctypes.byref(a), N.stream_handle(dev))
         if rc != N.LA_ERR_UNSUPPORTED:
             N.check(rc, "quest_select_hip")
             return ids, counts

@@ -573,11 +573,13 @@ int la_block_means(const la_block_means_args *a, void *stream);
  * (D a multiple of 8) score on the fp64 matrix cores first (for stride ==
  * block the antidiagonal entries pair query rows i mod block with key rows
  * -i mod block: block dense gram products per head, in-order fp64
- * accumulation over d, the same bits) and the selection reads the slots from
- * the workspace; otherwise the selection kernel scores every slot itself.
+ * accumulation over d, the same bits; bf16 rows of 64 or 128 values, with 256 or
+ * more key blocks, as exact sums of int8 limb products) and the selection reads the
+ * slots from the workspace; otherwise the selection kernel scores every slot itself.
  * The slots of a chunk of query blocks are scored and then selected, chunk
  * after chunk: la_xattn_select_workspace() sizes the chunk so that its slots
- * take at most 256 MiB (at least one chunk of 64 query blocks), and a smaller
+ * take at most 256 MiB (at least one chunk of 64 query blocks) and adds 4 * D bytes
+ * for each key row and each query row of a chunk where limbs are used; a smaller
  * workspace (B*Hq*64*n_kb*n_slots*8 bytes or more) gives smaller chunks with
  * the same lists.  la_xattn_select_workspace() returns 0 when no workspace
  * is used.

@@ -78,6 +78,9 @@ struct XaKP {
   // the launch covers query blocks [qc0, qc0 + n_qc) (rows (b, h, qb) of
   // that range, numbered b, h, qb - qc0 within the launch)
   int64_t qc0, n_qc;
+  // tiles left to the fp64 slot kernel, [b][h][64 query blocks][64 key blocks]
+  // (null: every tile)
+  uint8_t *left;
 };
 
 __device__ __forceinline__ uint64_t block_sum_u64(uint64_t v, uint64_t *red) {
@@ -161,6 +164,7 @@ __global__ __launch_bounds__(XM_NT, 3) void xattn_slots_mfma_kernel(XaKP p) {
   if (qb0 >= qend) return;
   const int64_t qlast = min(qb0 + XM_T, qend) - 1;
   if (kb0 * blk > qlast * blk + p.offset) return;  // every key block past causality
+  if (p.left && !p.left[(bh * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x]) return;
   const uint16_t *qbase = (const uint16_t *)p.q + b * p.q_sb + h * p.q_sh;
   const uint16_t *kbase = (const uint16_t *)p.k + b * p.k_sb + kvh * p.k_sh;
   // slice loads: chunk c (< 512) is row c / 8, 16-byte chunk c % 8, for the
@@ -268,6 +272,386 @@ __global__ __launch_bounds__(XM_NT, 3) void xattn_slots_mfma_kernel(XaKP p) {
   store(slot1, 1);
 }
 
+// The same slots on the int8 matrix cores, exact, for bf16 rows of 64 or 128
+// values: each row is a common exponent and integers X = m 2^(e - emin), |X| <
+// 2^(8 + R) with R the row's exponent range, written as balanced base-256 digits
+// (four for R <= 22, the top one zero for R <= 14).  An entry is then the integer
+// sum of its limb products, scaled by a power of two, and equals the sequential
+// fp64 sum of the (exact) bf16 products whenever every partial sum of that is
+// exact.  Partial sums are multiples of the least product bit and at most |Xq| |Xk|
+// of it (Cauchy-Schwarz, of any part of the rows), so |Xq| |Xk| <= 2^53 is enough; a
+// bound by the exponent ranges alone (128 * 2^(16 + Rq + Rk)) fails ten times as
+// many pairs of normal values.  Pairs outside the bound, and rows with an inf, a
+// NaN or R > 22, take the sequential fp64 sum; a tile with many of those is left
+// to the fp64 kernel.  The entries of slot 1 are added in fp64 in the same order
+// as there.
+//
+// xattn_limb_kernel: one workgroup per 16 rows of one residue mod block (the
+// rows (16 g + r) * blk + res of one head), 16 lanes a row; limbs go to the
+// matrix cores' operand order (row l % 16, values 16 (l / 16) .. + 15 of 64), a
+// word per row holds emin + 1024 and 4 log2 |X| rounded up (bits 16 on), a word per
+// 16 rows their largest of that and whether one has R > 14 (bit 16).
+constexpr int XI_NOLIMB = 1000, XI_EXACT = 4 * 53;
+struct XiRun {
+  const uint16_t *src;
+  int64_t sb, sh, st, H, T, blk, t0;  // t0: first row of the run (a multiple of blk)
+  int8_t *limbs;
+  int32_t *xw, *m16;
+  int32_t n16;  // 16-row groups per residue
+};
+template <int DH>
+__global__ __launch_bounds__(256) void xattn_limb_kernel(XiRun p) {
+  constexpr int EL = 4 * DH;  // values of a lane
+  const int tid = threadIdx.x, j = tid & 15, r = tid >> 4;
+  const int64_t g = blockIdx.x, res = blockIdx.y, bh = blockIdx.z;
+  const int64_t b = bh / p.H, h = bh % p.H;
+  const int64_t t = p.t0 + (16 * g + r) * p.blk + res;
+  uint32_t raw[EL / 2];
+#pragma unroll
+  for (int x = 0; x < EL / 2; ++x) raw[x] = 0u;
+  if (t < p.T) {
+    const uint16_t *row = p.src + b * p.sb + h * p.sh + t * p.st + EL * j;
+    if constexpr (DH == 2) {
+      const uint4 v = *(const uint4 *)row;
+      raw[0] = v.x; raw[1] = v.y; raw[EL / 2 - 2] = v.z; raw[EL / 2 - 1] = v.w;
+    } else {
+      const uint2 v = *(const uint2 *)row;
+      raw[0] = v.x; raw[1] = v.y;
+    }
+  }
+  int m[EL], e[EL];
+  int emin = 1 << 20, emax = -1, special = 0;
+#pragma unroll
+  for (int u = 0; u < EL; ++u) {
+    const uint32_t x = (raw[u >> 1] >> (16 * (u & 1))) & 0xffffu;
+    const uint32_t E = (x >> 7) & 0xffu, f = x & 0x7fu;
+    m[u] = E ? (int)(128u + f) : (int)f;
+    e[u] = E ? (int)E : 1;
+    special |= E == 255u;
+    if (m[u] != 0) {
+      emin = min(emin, e[u]);
+      emax = max(emax, e[u]);
+    }
+    if (x >> 15) m[u] = -m[u];
+  }
+#pragma unroll
+  for (int o = 8; o >= 1; o >>= 1) {  // over the row's 16 lanes
+    emin = min(emin, __shfl_xor(emin, o, 64));
+    emax = max(emax, __shfl_xor(emax, o, 64));
+    special |= __shfl_xor(special, o, 64);
+  }
+  if (emax < 0) emin = emax = 0;  // all zero
+  const int R = emax - emin;
+  const bool nolimb = special || R > 22;
+  double sq = 0.0;  // |X|^2
+  uint32_t word[4][DH];
+#pragma unroll
+  for (int l = 0; l < 4; ++l)
+#pragma unroll
+    for (int x = 0; x < DH; ++x) word[l][x] = 0u;
+#pragma unroll
+  for (int u = 0; u < EL; ++u) {
+    int X = nolimb || m[u] == 0 ? 0 : m[u] * (1 << (e[u] - emin));  // |X| < 2^30
+    sq += (double)X * (double)X;
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+      const int di = ((X + 128) & 255) - 128;
+      word[l][u / 4] |= (uint32_t)(di & 255) << (8 * (u & 3));
+      X = (X - di) >> 8;
+    }
+  }
+  const int64_t grp = (bh * p.blk + res) * p.n16 + g;
+  // value d = EL j .. + EL - 1: half d / 64, lane position r + 16 ((d % 64) / 16)
+  const int d0 = EL * j, pos = r + 16 * ((d0 & 63) >> 4);
+  int8_t *dst = p.limbs + grp * (DH * 4096) + (d0 >> 6) * 1024 + pos * 16 + (d0 & 15);
+#pragma unroll
+  for (int l = 0; l < 4; ++l)
+#pragma unroll
+    for (int x = 0; x < DH; ++x) *(uint32_t *)(dst + l * (DH * 1024) + 4 * x) = word[l][x];
+#pragma unroll
+  for (int o = 8; o >= 1; o >>= 1) sq += __shfl_xor(sq, o, 64);
+  // (the margin covers log2's and the sum's rounding)
+  const int L = nolimb ? XI_NOLIMB : sq > 0.0 ? (int)ceilf(2.f * log2f((float)sq) + 0.05f) : 0;
+  __shared__ int32_t s_m[16];
+  if (j == 0) {
+    p.xw[grp * 16 + r] = (emin + 1024) | (L << 16);
+    s_m[r] = L | (!nolimb && R > 14 ? 1 << 16 : 0);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    int mx = 0, big = 0;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      mx = max(mx, s_m[x] & 0xffff);
+      big |= s_m[x] >> 16;
+    }
+    p.m16[grp] = mx | (big << 16);
+  }
+}
+
+struct XiKP {
+  const int8_t *lq, *lk;
+  const int32_t *xq, *xk, *mq, *mk;
+  int32_t nq16, nk16;  // 16-row groups per residue (of the chunk's queries, of the keys)
+};
+
+// Tiles as in the fp64 kernel: 64 query x 64 key blocks, four waves of 32 x 32
+// (2 x 2 sub-tiles of 16 x 16).  A stage is one residue's 64 dims: 32 KiB of limbs
+// copied by LDS-DMA into one of two buffers while the other is multiplied (two
+// workgroups per CU); limb 3 of a 16-row group is copied and multiplied only
+// where its rows need it.  The sums of a residue stay in registers over its
+// stages.  Residue 0 comes last, so both slots of a pair leave together.
+// Everything a stage asks about its rows (fourth limbs, sub-tiles with a pair
+// outside the bound, exponents) is read once, into scalar masks and LDS: read in
+// the stages it was a chain of five memory latencies each, 838 us of this kernel
+// against 594, and 390 with the heads spread over the XCDs, so that a KV head's
+// limbs stay in one L2 (1.8 GB of limbs are read over all tiles).  The pairs
+// outside the bound are listed and summed first, a thread each; a tile of more than
+// XI_LIST of them, or with half of a wave's sub-tiles outside, is left.  1024 x 1024 blocks of 8 tokens, 32 heads, D = 128: 1209
+// us in the fp64 kernel (37 % of that matrix rate), 390 us here (the products take
+// 73 at the matrix rate: it waits for the copies of each stage), 68 for the limbs
+// and 14 to find no tile left.  Data that leave every tile pay 105 us for the try.
+constexpr int XI_LIST = 640, XI_BLK = 16;
+template <int DH>
+__global__ __launch_bounds__(XM_NT, 2) void xattn_slots_i8_kernel(XaKP p, XiKP x) {
+  typedef int v4i __attribute__((ext_vector_type(4)));
+  __shared__ __align__(16) int8_t sl[2][2][4][4][1024];  // [buffer][k, q][group][limb]
+  __shared__ __align__(16) int32_t s_x[2][XI_BLK][XM_T];  // row words [k, q][residue]
+  __shared__ double s_dot[XI_LIST];
+  __shared__ uint16_t s_pair[XI_LIST];  // 64 * key row + query row
+  __shared__ int32_t s_end[XI_BLK + 1];  // a residue's pairs: from s_end[i] on, then up to there
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g4 = lane >> 4, c16 = lane & 15;
+  int tx = (int)blockIdx.x, ty = (int)blockIdx.y, tz = (int)blockIdx.z;
+  if (gridDim.z % 8 == 0) {  // eight runs of heads, one per XCD
+    const uint32_t nxy = gridDim.x * gridDim.y, id = (uint32_t)tz * nxy + (uint32_t)ty * gridDim.x + (uint32_t)tx;
+    const uint32_t at = (id % 8) * (nxy * (gridDim.z / 8)) + id / 8, xy = at % nxy;
+    tz = (int)(at / nxy);
+    ty = (int)(xy / gridDim.x);
+    tx = (int)(xy % gridDim.x);
+  }
+  const int64_t kb0 = (int64_t)tx * XM_T, ql0 = (int64_t)ty * XM_T;  // ql0: in the chunk
+  const int64_t bh = tz, b = bh / p.Hq, h = bh % p.Hq, kvh = h / (p.Hq / p.Hkv);
+  const int64_t qlast = p.qc0 + min(ql0 + XM_T, p.n_qc) - 1;
+  if (kb0 * p.blk > qlast * p.blk + p.offset) return;  // every key block past causality
+  uint8_t *const left = p.left + (bh * gridDim.y + ty) * gridDim.x + tx;
+  const int blk = (int)p.blk, n16k = x.nk16, n16q = x.nq16;
+  // the k row of residue i's query row is residue (blk - i) % blk
+  const int64_t qg0 = bh * blk * n16q + ql0 / 16, kg0 = (b * p.Hkv + kvh) * blk * n16k + kb0 / 16;
+  auto kres = [&](int i) { return i ? blk - i : 0; };
+  const int kw = w & 1, qw = w >> 1;
+  // lane l: the groups l % 4 of residue l / 4, then its sub-tile l % 4 of this wave
+  const int li = lane >> 2;
+  const bool lv = li < blk;
+  const int32_t mk1 = lv ? x.mk[kg0 + (int64_t)kres(li) * n16k + (lane & 3)] : 0;
+  const int32_t mq1 = lv ? x.mq[qg0 + (int64_t)li * n16q + (lane & 3)] : 0;
+  const int kg1 = 2 * kw + ((lane >> 1) & 1), qg1 = 2 * qw + (lane & 1);
+  const int32_t lk1 = __shfl(mk1, (lane & ~3) + kg1, 64) & 0xffff;
+  const int32_t lq1 = __shfl(mq1, (lane & ~3) + qg1, 64) & 0xffff;
+  const uint64_t kbig = __ballot(mk1 >> 16), qbig = __ballot(mq1 >> 16);
+  const uint64_t bad = __ballot(lv && lk1 + lq1 > XI_EXACT);  // [residue][key group][query group]
+  for (int y = tid; y < blk * 2 * XM_T; y += XM_NT) {
+    const int i = y >> 7, side = (y >> 6) & 1, r = y & 63;
+    s_x[side][i][r] = side == 0 ? x.xk[(kg0 + (int64_t)kres(i) * n16k) * 16 + r]
+                                : x.xq[(qg0 + (int64_t)i * n16q) * 16 + r];
+  }
+  if (tid <= XI_BLK) s_end[tid] = 0;
+  if (__syncthreads_or(bad != 0)) {
+    // over the wave's sub-tiles with such pairs: fn(residue, key row, query row)
+    auto pairs = [&](auto fn) {
+      for (uint64_t m = bad; m; m &= m - 1) {
+        const int y = __builtin_ctzll(m), i = y >> 2;
+        const int r0 = 32 * kw + 8 * (y & 2) + 4 * g4, c = 32 * qw + 16 * (y & 1) + c16;
+        const int xq = s_x[1][i][c] >> 16;
+        for (int e = 0; e < 4; ++e)
+          if ((s_x[0][i][r0 + e] >> 16) + xq > XI_EXACT) fn(i, r0 + e, c);
+      }
+    };
+    const bool many = __syncthreads_or(__popcll(bad) > 2 * blk);  // half of a wave's sub-tiles: not counted
+    if (!many) pairs([&](int i, int, int) { atomicAdd(&s_end[i + 1], 1); });
+    __syncthreads();
+    int n = 0, start = 0;
+    for (int i = 0; i < blk; ++i) {
+      if (i == tid) start = n;
+      n += s_end[i + 1];
+    }
+    const bool leave = many || n > XI_LIST;
+    if (tid == 0) *left = leave;
+    if (leave) return;
+    __syncthreads();
+    if (tid < blk) s_end[tid + 1] = start;
+    __syncthreads();
+    pairs([&](int i, int r, int c) { s_pair[atomicAdd(&s_end[i + 1], 1)] = (uint16_t)(64 * r + c); });
+    __syncthreads();  // s_end[i + 1]: the end of residue i's, and the start of the next's
+    for (int y = tid; y < n; y += XM_NT) {
+      int i = 0;
+      while (s_end[i + 1] <= y) ++i;
+      const int64_t tq = (p.qc0 + ql0 + (s_pair[y] & 63)) * blk + i, tk = (kb0 + (s_pair[y] >> 6)) * blk + kres(i);
+      const uint4 *qr = (const uint4 *)((const uint16_t *)p.q + b * p.q_sb + h * p.q_sh + tq * p.q_st);
+      const uint4 *kr = (const uint4 *)((const uint16_t *)p.k + b * p.k_sb + kvh * p.k_sh + tk * p.k_st);
+      double a = 0.0;
+#pragma unroll 1
+      for (int d = 0; d < DH; ++d) {
+        uint4 qv[8], kv[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {  // (rows past the end are zeros, also against an inf)
+          qv[c] = kv[c] = uint4{0u, 0u, 0u, 0u};
+          if (tq < p.Tq) qv[c] = qr[8 * d + c];
+          if (tk < p.T) kv[c] = kr[8 * d + c];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all in flight
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const uint32_t q4[4] = {qv[c].x, qv[c].y, qv[c].z, qv[c].w};
+          const uint32_t k4[4] = {kv[c].x, kv[c].y, kv[c].z, kv[c].w};
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            a = __builtin_fma((double)bf16lo(k4[u]), (double)bf16lo(q4[u]), a);
+            a = __builtin_fma((double)bf16hi(k4[u]), (double)bf16hi(q4[u]), a);
+          }
+        }
+      }
+      s_dot[y] = a;
+    }
+    __syncthreads();
+  } else if (tid == 0) {
+    *left = 0;
+  }
+  // wave w copies groups 2 (w % 2), + 1 of k (w < 2) or q
+  const int side = w >> 1, gb = 2 * (w & 1);
+  const int8_t *const src0 = (side == 0 ? x.lk + kg0 * (DH * 4096) : x.lq + qg0 * (DH * 4096)) + lane * 16;
+  const uint64_t sbig = side == 0 ? kbig : qbig;
+  auto copy = [&](int i, int dh, int buf) {
+    const int8_t *src = src0 + (int64_t)(side == 0 ? kres(i) * n16k + gb : i * n16q + gb) * (DH * 4096) + dh * 1024;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int l = 0; l < 3; ++l) dma16(src + (u * 4 + l) * (DH * 1024), &sl[buf][side][gb + u][l][0]);
+      if ((sbig >> (4 * i + gb + u)) & 1) dma16(src + (u * 4 + 3) * (DH * 1024), &sl[buf][side][gb + u][3][0]);
+    }
+  };
+  double slot1[2][2][4];
+#pragma unroll
+  for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) slot1[ib][jb][e] = 0.0;
+  const int i0 = blk > 1 ? 1 : 0;  // residues 1 .. blk - 1, then 0
+  copy(i0, 0, 0);
+  int buf = 0;
+#pragma unroll 1
+  for (int s = 0, i = i0; s < blk; ++s, i = i + 1 < blk ? i + 1 : 0) {
+    const int next = i + 1 < blk ? i + 1 : 0;
+    const uint32_t kb2 = (uint32_t)(kbig >> (4 * i + 2 * kw)) & 3u, qb2 = (uint32_t)(qbig >> (4 * i + 2 * qw)) & 3u;
+    v4i acc[2][2][7];
+#pragma unroll
+    for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+        for (int g = 0; g < 7; ++g) acc[ib][jb][g] = v4i{0, 0, 0, 0};
+#pragma unroll 1
+    for (int dh = 0; dh < DH; ++dh, buf ^= 1) {
+      wait_vmcnt<0>();  // this wave's copies of the stage
+      __syncthreads();  // every wave's; the other buffer is read
+      if (dh + 1 < DH)
+        copy(i, dh + 1, buf ^ 1);
+      else if (s + 1 < blk)
+        copy(next, 0, buf ^ 1);
+      v4i A[2][4], B[2][4];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int l = 0; l < 3; ++l) {
+          A[u][l] = *(const v4i *)&sl[buf][0][2 * kw + u][l][lane * 16];
+          B[u][l] = *(const v4i *)&sl[buf][1][2 * qw + u][l][lane * 16];
+        }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if ((kb2 >> u) & 1) A[u][3] = *(const v4i *)&sl[buf][0][2 * kw + u][3][lane * 16];
+        if ((qb2 >> u) & 1) B[u][3] = *(const v4i *)&sl[buf][1][2 * qw + u][3][lane * 16];
+      }
+      auto mul = [&](int ib, int jb, int la, int lb) {
+        acc[ib][jb][la + lb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[ib][la], B[jb][lb], acc[ib][jb][la + lb], 0, 0, 0);
+      };
+#pragma unroll
+      for (int la = 0; la < 3; ++la)
+#pragma unroll
+        for (int lb = 0; lb < 3; ++lb)
+#pragma unroll
+          for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+            for (int jb = 0; jb < 2; ++jb) mul(ib, jb, la, lb);
+#pragma unroll
+      for (int ib = 0; ib < 2; ++ib)
+        if ((kb2 >> ib) & 1) {
+#pragma unroll
+          for (int jb = 0; jb < 2; ++jb) {
+#pragma unroll
+            for (int lb = 0; lb < 3; ++lb) mul(ib, jb, 3, lb);
+            if ((qb2 >> jb) & 1) mul(ib, jb, 3, 3);
+          }
+        }
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb)
+        if ((qb2 >> jb) & 1) {
+#pragma unroll
+          for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+            for (int la = 0; la < 3; ++la) mul(ib, jb, la, 3);
+        }
+    }
+    // the residue's entries: lane holds key rows 4 g4 + e of its key groups and
+    // query row c16 of its query groups
+#pragma unroll
+    for (int ib = 0; ib < 2; ++ib)
+#pragma unroll
+      for (int jb = 0; jb < 2; ++jb) {
+        const int r0 = 32 * kw + 16 * ib + 4 * g4, c = 32 * qw + 16 * jb + c16;
+        const int4 xk = *(const int4 *)&s_x[0][i][r0];
+        const int xq = (s_x[1][i][c] & 0xffff) - 2048 - 268;
+        const int xe[4] = {(xk.x & 0xffff) + xq, (xk.y & 0xffff) + xq, (xk.z & 0xffff) + xq, (xk.w & 0xffff) + xq};
+        const bool big = ((kb2 >> ib) | (qb2 >> jb)) & 1;  // (wave-uniform)
+        double dot[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // lo + m1 2^16 + m2 2^32 + top 2^48, each part within int32
+          const v4i *a = acc[ib][jb];
+          const int32_t lo = a[0][e] + a[1][e] * 256, m1 = a[2][e] + a[3][e] * 256;
+          double v;
+          if (big) {
+            v = (double)a[6][e];
+            v = __builtin_fma(v, 65536.0, (double)(a[4][e] + a[5][e] * 256));
+          } else {
+            v = (double)a[4][e];
+          }
+          v = __builtin_fma(v, 65536.0, (double)m1);
+          v = __builtin_fma(v, 65536.0, (double)lo);
+          dot[e] = __builtin_amdgcn_ldexp(v, xe[e]);
+        }
+        if ((bad >> (4 * i + 2 * ib + jb)) & 1)
+          for (int y = s_end[i]; y < s_end[i + 1]; ++y) {
+            const int at = s_pair[y] - (64 * r0 + c);
+            const double a = s_dot[y];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dot[e] = at == 64 * e ? a : dot[e];
+          }
+        if (i != 0) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) slot1[ib][jb][e] = slot1[ib][jb][e] + dot[e];
+        } else {  // both slots of the lane's four pairs: 64 bytes, 256 per query row
+          const int64_t ql = ql0 + c, kb = kb0 + r0;
+          double2 *out = (double2 *)p.slots + (bh * p.n_qc + ql) * p.n_kb + kb;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (ql < p.n_qc && kb + e < p.n_kb)
+              out[e] = double2{(0.0 + dot[e]) * p.inv_sqrt_d, slot1[ib][jb][e] * p.inv_sqrt_d};
+        }
+      }
+  }
+}
 template <int KPT>
 __global__ __launch_bounds__(TK_NT) void xattn_select_kernel(XaKP p) {
   extern __shared__ __align__(16) unsigned char dyn[];
@@ -705,13 +1089,59 @@ static int xattn_launch_select(const XaKP &p, int64_t n_kb, size_t lds, int64_t 
   return LA_OK;
 }
 
+// The int8 form: bf16 rows of 64 or 128 values (its row words and limbs, 4 * D
+// bytes a row, come on top of the slots), four or more tiles of keys and enough
+// tiles for two workgroups per CU.  The limb pass and the further launches are
+// paid back over the tiles that a row is multiplied with, and fp64 tiles run side
+// by side until the chip is full.  Whole calls, 32 heads, D = 128, blocks of 8, us
+// (int8, fp64): 256 blocks 152, 164; 128 blocks 113, 97 (batch 4: 207, 193);
+// 64 blocks 92, 83; with 4 heads at 256 blocks 92, 85.
+struct XiLayout {
+  size_t lk, xk, mk, lq, xq, mq, left, bytes;
+  int64_t nk16, nq16;
+};
+static bool xattn_i8_shape(const la_xattn_select_args *a) {
+  const int64_t n_kb = ceil_div(a->T, a->block), n_qb = ceil_div(a->Tq, a->block);
+  return xattn_mfma_shape(a) && a->in_dtype == LA_BF16 && (a->D == 64 || a->D == 128) && a->block <= XI_BLK &&
+         n_kb >= 4 * XM_T && n_qb >= XM_T && a->B * a->Hq * ceil_div(n_qb, XM_T) * ceil_div(n_kb, XM_T) >= 512 &&
+         a->B * a->Hkv * ceil_div(a->T, a->block) * a->block * a->D * 4 <= ((int64_t)256 << 20);
+}
+static XiLayout xattn_i8_layout(const la_xattn_select_args *a, int64_t cq) {
+  XiLayout L{};
+  L.nk16 = ceil_div(ceil_div(a->T, a->block), XM_T) * (XM_T / 16);
+  L.nq16 = ceil_div(cq, XM_T) * (XM_T / 16);
+  const int64_t gk = a->B * a->Hkv * a->block * L.nk16, gq = a->B * a->Hq * a->block * L.nq16;
+  size_t at = ((size_t)xattn_slot_bytes(a, cq) + 255) / 256 * 256;
+  auto take = [&](int64_t n) {
+    const size_t o = at;
+    at += ((size_t)n + 255) / 256 * 256;
+    return o;
+  };
+  L.lk = take(gk * 64 * a->D);
+  L.xk = take(gk * 64);
+  L.mk = take(gk * 4);
+  L.lq = take(gq * 64 * a->D);
+  L.xq = take(gq * 64);
+  L.mq = take(gq * 4);
+  L.left = take(a->B * a->Hq * (L.nq16 / 4) * (L.nk16 / 4));
+  L.bytes = at;
+  return L;
+}
+// Query blocks per launch of the int8 form within `avail` bytes (0: not even XM_T).
+static int64_t xattn_i8_chunk(const la_xattn_select_args *a, int64_t avail) {
+  const int64_t n_qb = ceil_div(a->Tq, a->block);
+  int64_t c = std::min(xattn_chunk_qb(a, avail), n_qb);
+  while (c > 0 && (int64_t)xattn_i8_layout(a, c).bytes > avail) c = (c - 1) / XM_T * XM_T;
+  return c;
+}
+
 extern "C" size_t la_xattn_select_workspace(const la_xattn_select_args *a) {
   if (!a || a->B <= 0 || a->Hq <= 0 || a->Tq <= 0 || a->T <= 0 || a->block < 1 || a->stride < 1)
     return 0;
   if (!xattn_mfma_shape(a)) return 0;
   const int64_t cq = std::max<int64_t>(xattn_chunk_qb(a, XA_SLOT_BUDGET),
                                        std::min<int64_t>(XM_T, ceil_div(a->Tq, a->block)));
-  return (size_t)xattn_slot_bytes(a, cq);
+  return xattn_i8_shape(a) ? xattn_i8_layout(a, cq).bytes : (size_t)xattn_slot_bytes(a, cq);
 }
 
 extern "C" int la_xattn_select(const la_xattn_select_args *a, void *stream) {
@@ -757,16 +1187,52 @@ extern "C" int la_xattn_select(const la_xattn_select_args *a, void *stream) {
   const int64_t nwg = a->B * a->Hq * n_qb;
   LA_REQUIRE(nwg < ((int64_t)1 << 31), "la_xattn_select: too many rows");
   hipStream_t st = (hipStream_t)stream;
-  const int64_t cq = a->workspace && xattn_mfma_shape(a) ? xattn_chunk_qb(a, a->ws_bytes) : 0;
+  // int8 where its limbs fit the workspace too and leave at least half the chunk, else fp64
+  const int64_t c64 = a->workspace && xattn_mfma_shape(a) ? xattn_chunk_qb(a, a->ws_bytes) : 0;
+  int64_t ci = c64 > 0 && (uintptr_t)a->workspace % 16 == 0 && xattn_i8_shape(a)
+                   ? xattn_i8_chunk(a, a->ws_bytes) : 0;
+  if (2 * ci < c64) ci = 0;
+  const int64_t cq = ci > 0 ? ci : c64;
   if (cq > 0) {
     p.slots = (double *)a->workspace;
     LA_REQUIRE(a->B * a->Hq < 65536, "la_xattn_select: B * Hq >= 65536");
+    char *ws = (char *)a->workspace;
+    const XiLayout L = ci > 0 ? xattn_i8_layout(a, cq) : XiLayout{};
+    XiKP x{(const int8_t *)(ws + L.lq), (const int8_t *)(ws + L.lk), (const int32_t *)(ws + L.xq),
+           (const int32_t *)(ws + L.xk), (const int32_t *)(ws + L.mq), (const int32_t *)(ws + L.mk),
+           (int32_t)L.nq16, (int32_t)L.nk16};
+    auto limbs = [&](const XiRun &r, int64_t heads) {
+      const dim3 g((unsigned)r.n16, (unsigned)a->block, (unsigned)(a->B * heads));
+      if (a->D == 128)
+        xattn_limb_kernel<2><<<g, 256, 0, st>>>(r);
+      else
+        xattn_limb_kernel<1><<<g, 256, 0, st>>>(r);
+    };
+    if (ci > 0) {
+      limbs(XiRun{(const uint16_t *)a->k, a->k_sb, a->k_sh, a->k_st, a->Hkv, a->T, a->block, 0,
+                  (int8_t *)(ws + L.lk), (int32_t *)(ws + L.xk), (int32_t *)(ws + L.mk), (int32_t)L.nk16},
+            a->Hkv);
+      LA_LAUNCHED();
+      p.left = (uint8_t *)(ws + L.left);
+    }
     // chunks of query blocks: score the chunk's slots, then select its rows
     for (int64_t q0 = 0; q0 < n_qb; q0 += cq) {
       p.qc0 = q0;
       p.n_qc = std::min(cq, n_qb - q0);
       const dim3 grid((unsigned)ceil_div(n_kb, XM_T), (unsigned)ceil_div(p.n_qc, XM_T),
                       (unsigned)(a->B * a->Hq));
+      if (ci > 0) {
+        limbs(XiRun{(const uint16_t *)a->q, a->q_sb, a->q_sh, a->q_st, a->Hq, a->Tq, a->block, q0 * a->block,
+                    (int8_t *)(ws + L.lq), (int32_t *)(ws + L.xq), (int32_t *)(ws + L.mq), (int32_t)L.nq16},
+              a->Hq);
+        LA_LAUNCHED();
+        if (a->D == 128)
+          xattn_slots_i8_kernel<2><<<grid, XM_NT, 0, st>>>(p, x);
+        else
+          xattn_slots_i8_kernel<1><<<grid, XM_NT, 0, st>>>(p, x);
+        LA_LAUNCHED();
+      }
+      // (after the int8 form: the tiles it left)
       if (a->in_dtype == LA_BF16)
         xattn_slots_mfma_kernel<true><<<grid, XM_NT, 0, st>>>(p);
       else

@@ -168,9 +168,10 @@ def xattn_select_hip(q: torch.Tensor, k: torch.Tensor, *, block: int = 8, stride
     function of the inputs (ties to the lowest block).
 
     The slot scores of a chunk of query blocks are kept in a workspace of at
-    most 256 MiB (the chunk shrinks as T grows); ``max_workspace_bytes``
-    bounds it further (smaller chunks, same lists; below one chunk of 64 query
-    blocks the rows are scored without a workspace).
+    most 256 MiB (the chunk shrinks as T grows), beside the int8 limbs of bf16
+    rows (4 * D bytes a row) for 256 or more key blocks; ``max_workspace_bytes``
+    bounds both (smaller chunks or no limbs, same lists; below one chunk of 64
+    query blocks the rows are scored without a workspace).
 
     q (B, Hq, Tq, D) at positions offset + t; k (B, Hkv, T, D).  Returns ids
     (B, Hq, n_qb, W) ascending, -1 padded (W = n_kb, or min(topk, n_kb) + 1)

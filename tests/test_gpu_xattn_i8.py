@@ -1,0 +1,51 @@
+"""XAttention's slots on the int8 matrix cores against the fp64 form.
+
+Both are exact sums in the same order, so the block lists must be identical, bit
+for bit.  A workspace of one run of 64 query blocks' slots has no room for limbs and
+takes the fp64 form.  The data decide what a pair takes: an exponent range within
+the bound (int8), a few rows past it (listed pairs), most rows past it (tiles left
+to the fp64 kernel), infs and NaN."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # B, Hq, Hkv, Tq, T, D, block, offset: from 256 key blocks and 512 tiles on
+    (1, 32, 8, 2048, 2048, 128, 8, 0),     # whole tiles; heads spread over XCDs
+    (2, 18, 2, 1030, 1030, 128, 4, 0),     # a partial last block and tile
+    (1, 36, 4, 530, 530, 64, 2, 0),
+    (2, 32, 8, 650, 2600, 64, 8, 1950),    # queries at an offset
+    (1, 24, 8, 1030, 4110, 128, 16, 3080),
+]
+
+
+@pytest.mark.parametrize("data", ["normal", "few", "wide", "special"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_int8_slots_select_as_fp64(shape, data):
+    from linattn_amd.kernels.routing import xattn_select_hip
+    B, Hq, Hkv, Tq, T, D, blk, off = shape
+    g = torch.Generator().manual_seed(T + D)
+    q = torch.randn(B, Tq, Hq, D, generator=g)
+    k = torch.randn(B, Hkv, T, D, generator=g)
+    if data == "few":  # rows of more than 23 octaves
+        q[:, 5::97, :, 0] = 3e7
+        k[:, :, 11::131, -1] = 1e-9
+    elif data == "wide":
+        q *= torch.exp(4 * torch.randn(q.shape, generator=g))
+        k *= torch.exp(4 * torch.randn(k.shape, generator=g))
+    elif data == "special":
+        q[:, 17] = 0.0
+        q[:, 30, :, 3] = float("inf")
+        k[:, :, 40, 5] = float("nan")
+        k[:, :, 41, 6] = -float("inf")
+        k[:, :, 50] = 1e-40  # denormal
+    q = q.bfloat16().cuda().transpose(1, 2)  # [B, Hq, Tq, D] over [B, Tq, Hq, D]
+    k = k.bfloat16().cuda()
+    n_kb = -(-T // blk)
+    for sel in (dict(threshold=0.9), dict(topk=7)):
+        kw = dict(block=blk, stride=blk, offset=off, **sel)
+        ids, counts = xattn_select_hip(q, k, **kw)
+        rids, rcounts = xattn_select_hip(q, k, max_workspace_bytes=B * Hq * 64 * n_kb * 2 * 8, **kw)
+        assert torch.equal(counts, rcounts)
+        assert torch.equal(ids, rids)

@@ -407,10 +407,11 @@ struct XiKP {
 // against 594, and 390 with the heads spread over the XCDs, so that a KV head's
 // limbs stay in one L2 (1.8 GB of limbs are read over all tiles).  The pairs
 // outside the bound are listed and summed first, a thread each; a tile of more than
-// XI_LIST of them, or with half of a wave's sub-tiles outside, is left.  1024 x 1024 blocks of 8 tokens, 32 heads, D = 128: 1209
-// us in the fp64 kernel (37 % of that matrix rate), 390 us here (the products take
-// 73 at the matrix rate: it waits for the copies of each stage), 68 for the limbs
-// and 14 to find no tile left.  Data that leave every tile pay 105 us for the try.
+// XI_LIST of them, or with half of a wave's sub-tiles outside, is left.  1024 x
+// 1024 blocks of 8 tokens, 32 heads, D = 128: 1209 us in the fp64 kernel (37 % of
+// that matrix rate), 390 us here (the products take 73 at the matrix rate: it waits
+// for the copies of each stage), 68 for the limbs and 14 to find no tile left.
+// Data that leave every tile pay 105 us for the try.
 constexpr int XI_LIST = 640, XI_BLK = 16;
 template <int DH>
 __global__ __launch_bounds__(XM_NT, 2) void xattn_slots_i8_kernel(XaKP p, XiKP x) {
@@ -881,32 +882,38 @@ __device__ __forceinline__ uint64_t wave_red_u64(uint64_t x) {
 // The selection of xattn_select_kernel for rows whose slot scores are already
 // in the workspace (stride == block) and that have at most 64 * KPL key
 // blocks: one wave per row, block kb = lane + 64 j in slot j of the lane's
-// registers, every reduction a lane exchange -- the ~40 steps of the
-// threshold search take no barrier.  The arithmetic (row maximum, masses,
-// the threshold and tie rules, top-k by (mass desc, block asc), the own
+// registers, every reduction a lane exchange -- the steps of the threshold
+// search take no barrier.  A step costs a compare and a 64-bit sum per register
+// and a wave reduction of some 200 clocks, and a search over every bit of a mass
+// takes 45: once at most 64 blocks are between the bounds (after about 12 steps
+// for 1024 normal scores) each lane takes one and the rest is one pass over 64
+// masses in LDS.  32 heads x 1024 rows of 1024 blocks: 416 us bit by bit with the
+// slots read twice, one pair at a time; 190 us here.  The arithmetic (row maximum,
+// masses, the threshold and tie rules, top-k by (mass desc, block asc), the own
 // block) is the block kernel's, so the lists are identical.
 template <int KPL>
 __global__ __launch_bounds__(256) void xattn_select_wave_kernel(XaKP p, int64_t n_rows) {
-  const int lane = threadIdx.x & 63;
+  __shared__ __align__(16) uint64_t s_left[4][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t lrow = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);  // (b, h, qb - qc0)
   if (lrow >= n_rows) return;  // wave-uniform; the kernel has no barrier
   const int64_t qb = p.qc0 + lrow % p.n_qc;
   const int64_t h = (lrow / p.n_qc) % p.Hq;
   const int64_t row = (lrow / (p.n_qc * p.Hq) * p.Hq + h) * p.n_qb + qb;  // the output row
-  const int64_t n_kb = p.n_kb, NS = p.n_slots, blk = p.blk;
+  const int64_t n_kb = p.n_kb, blk = p.blk;
   const int64_t pos0 = qb * blk + p.offset;
   const int64_t lim = min(pos0 / blk, n_kb - 1);
   const int64_t n_vis = lim + 1;
-  const double *src = p.slots + lrow * n_kb * NS;
+  const double2 *src = (const double2 *)p.slots + lrow * n_kb;  // both slots of a block
   const uint64_t lt = lanemask_lt(lane);
 
+  double2 sc[KPL];
+#pragma unroll
+  for (int j = 0; j < KPL; ++j) sc[j] = src[min(lane + 64 * (int64_t)j, lim)];  // all in flight
   double mx = __int_as_float(0xff800000);
 #pragma unroll
-  for (int j = 0; j < KPL; ++j) {
-    const int64_t kb = lane + 64 * j;
-    if (kb < n_vis)
-      for (int64_t s = 0; s < NS; ++s) mx = fmax(mx, src[kb * NS + s]);
-  }
+  for (int j = 0; j < KPL; ++j)
+    if (lane + 64 * (int64_t)j < n_vis) mx = fmax(fmax(mx, sc[j].x), sc[j].y);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
 
@@ -917,7 +924,8 @@ __global__ __launch_bounds__(256) void xattn_select_wave_kernel(XaKP p, int64_t 
     const int64_t kb = lane + 64 * j;
     uint64_t m = 0;
     if (kb < n_vis)
-      for (int64_t s = 0; s < NS; ++s) m += (uint64_t)__builtin_rint(exp_det(src[kb * NS + s] - mx) * p.two_f);
+      m = (uint64_t)__builtin_rint(exp_det(sc[j].x - mx) * p.two_f) +
+          (uint64_t)__builtin_rint(exp_det(sc[j].y - mx) * p.two_f);
     u[j] = m;
     zpart += m;
     umax = m > umax ? m : umax;
@@ -944,14 +952,53 @@ __global__ __launch_bounds__(256) void xattn_select_wave_kernel(XaKP p, int64_t 
     } else {
       const uint64_t thr = (uint64_t)ceil(thr_d);
       // largest v with sum(mass >= v) >= thr (v = 0 qualifies: the sum is Z)
-      uint64_t v = 0;
-      for (int bit = top ? 63 - __clzll((long long)top) : -1; bit >= 0; --bit) {
+      uint64_t v = 0, v_hi = ~0ull, s_hi = 0;  // the answer is in [v, v_hi); s_hi = sum(mass >= v_hi)
+      int n_lo = 64 * jn, n_hi = 0;            // blocks >= v, blocks >= v_hi
+      for (int bit = top ? 63 - __clzll((long long)top) : -1; bit >= 0 && n_lo - n_hi > 64; --bit) {
         const uint64_t v2 = v | (1ull << bit);
         uint64_t part = 0;
+        int n = 0;
 #pragma unroll
         for (int j = 0; j < KPL; ++j)
-          if (j < jn) part += u[j] >= v2 ? u[j] : 0ull;
-        if (wave_red_u64<false>(part) >= thr) v = v2;
+          if (j < jn) {
+            const bool ge = u[j] >= v2;
+            part += ge ? u[j] : 0ull;
+            n += __popcll(__ballot(ge));
+          }
+        part = wave_red_u64<false>(part);
+        if (part >= thr) {
+          v = v2;
+          n_lo = n;
+        } else {
+          v_hi = v2;
+          s_hi = part;
+          n_hi = n;
+        }
+      }
+      if (n_lo - n_hi <= 64) {
+        // at most a block per lane is left, and the answer is one of their masses
+        // (thr > 0): each lane sums the masses not below its own
+        s_left[w][lane] = 0;
+        int at = 0;
+#pragma unroll
+        for (int j = 0; j < KPL; ++j)
+          if (j < jn) {
+            const bool in = u[j] >= v && u[j] < v_hi;
+            const uint64_t bm = __ballot(in);
+            if (in) s_left[w][at + __popcll(bm & lt)] = u[j];
+            at += __popcll(bm);
+          }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // one wave writes and reads these
+        const uint64_t mine = s_left[w][lane];
+        uint64_t sum = s_hi;
+        for (int y = 0; y < at; y += 4) {
+          uint64_t m[4];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) m[c] = s_left[w][y + c];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) sum += m[c] >= mine ? m[c] : 0ull;
+        }
+        v = wave_red_u64<true>(sum >= thr ? mine : 0ull);
       }
       uint64_t gpart = 0;
 #pragma unroll

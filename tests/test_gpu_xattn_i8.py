@@ -49,3 +49,29 @@ def test_int8_slots_select_as_fp64(shape, data):
         rids, rcounts = xattn_select_hip(q, k, max_workspace_bytes=B * Hq * 64 * n_kb * 2 * 8, **kw)
         assert torch.equal(counts, rcounts)
         assert torch.equal(ids, rids)
+
+
+@pytest.mark.parametrize("data", ["equal", "levels", "normal", "steep"])
+@pytest.mark.parametrize("n_kb", [1, 64, 65, 130, 300, 1000])
+def test_threshold_search_of_one_wave(n_kb, data):
+    """The wave's search (bits, then the last 64 blocks at once) keeps what the
+    workgroup's bitwise search keeps: more than 64 equal masses (never down to a
+    block per lane), a few levels of equal masses, and no two equal."""
+    from linattn_amd.kernels.routing import xattn_select_hip
+    g = torch.Generator().manual_seed(n_kb)
+    q = torch.randn(1, 2, 2 * n_kb, 16, generator=g)
+    k = torch.randn(1, 1, 2 * n_kb, 16, generator=g)
+    if data == "equal":
+        q.zero_()
+    elif data == "levels":
+        q.fill_(0.5)
+        k = torch.randint(0, 3, (1, 1, 2 * n_kb, 1), generator=g).float().expand(k.shape).contiguous()
+    elif data == "steep":
+        q *= 20
+    q, k = q.half().cuda(), k.half().cuda()
+    for thr in (0.02, 0.5, 0.9, 0.9999999, 1.0):
+        kw = dict(block=2, stride=2, threshold=thr)
+        ids, counts = xattn_select_hip(q, k, **kw)
+        rids, rcounts = xattn_select_hip(q, k, max_workspace_bytes=0, **kw)
+        assert torch.equal(counts, rcounts)
+        assert torch.equal(ids, rids)

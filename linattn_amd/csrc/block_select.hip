@@ -152,7 +152,7 @@ __device__ __forceinline__ double sc_widen(const uint4 &v, int i) {
 // heads on 64 blocks, D = 128: 59 us with the widening pass and 4 x 4 scores per
 // thread, 27 like this.  Rows of 8-byte values (pooled q) need four times as many
 // scattered loads and stay with block_score_kernel (64 heads of 512 x 512, causal:
-// 208 us there, 205-290 in forms of this one).
+// 144 us there, 205-290 in forms of this one).
 template <int DT, int R>
 __global__ __launch_bounds__(256) void row_score_kernel(ScKP p) {
   constexpr int EV = DT == LA_F32 ? 4 : 8;  // values of a 16-byte load
@@ -261,15 +261,25 @@ __global__ __launch_bounds__(256) void few_row_score_kernel(ScKP p) {
 }
 
 // Any shape (and pooled q, F64): 4 x 4 scores per thread on 64 x 64 tiles staged
-// in LDS.
+// in LDS.  VEC (pooled q and means in 16-byte pieces): the next 32 dims are in
+// flight, all loads at once, while these are multiplied (loaded one by one between
+// two barriers they took longer than the products).  Bound by the fp64 instructions
+// (a multiply and an add per product) and as many LDS clocks.  64 heads of 512 x 512
+// on 128 dims, causal: 203 us loaded one by one, 157 loaded ahead, 144 with columns
+// read in runs of 256 bytes and whole slices unrolled (56 for the instructions; held
+// to 128 registers for a fourth workgroup per CU it spills and takes 168).
 constexpr int BS_DC = 32, BS_NT = 256;
-template <bool F64>
+template <bool F64, bool VEC>
 __global__ __launch_bounds__(BS_NT) void block_score_kernel(ScKP p) {
   constexpr int TQ = 64, RQ = 4, RK = 4, TX = BS_NT / (TQ / RQ), TK = TX * RK;
-  __shared__ double sq[BS_DC][TQ + 2];
-  __shared__ double sk[BS_DC][TK + 2];
+  constexpr int NV = TQ * BS_DC / (2 * BS_NT);  // pairs of a thread's share of a slice
+  static_assert(TQ == TK && (!VEC || F64), "");
+  __shared__ __align__(16) double sq[BS_DC][TQ + 2];
+  __shared__ __align__(16) double sk[BS_DC][TK + 2];
   const int tid = threadIdx.x;
-  const int tq = tid / TX, tk = tid % TX;  // rows RQ*tq.., cols RK*tk..
+  // rows RQ*tq.., columns 2*tk, 2*tk + 1 and TK/2 on: 16 threads read 256 bytes in a row
+  const int tq = tid / TX, tk = tid % TX;
+  auto col = [&](int c) { return (c >> 1) * (TK / 2) + 2 * tk + (c & 1); };
   const int64_t i0 = (int64_t)blockIdx.y * TQ, j0 = (int64_t)blockIdx.x * TK;
   const int64_t bh = blockIdx.z;
   const int64_t b = bh / p.Hq, h = bh % p.Hq;
@@ -281,31 +291,62 @@ __global__ __launch_bounds__(BS_NT) void block_score_kernel(ScKP p) {
   for (int a = 0; a < RQ; ++a)
 #pragma unroll
     for (int c = 0; c < RK; ++c) acc[a][c] = 0.0;
+  double2 vq[NV], vk[NV];
+  // (rows and dims past the end read the last ones; their sums are not stored or not formed)
+  auto fetch = [&](int64_t d0) {
+#pragma unroll
+    for (int x = 0; x < NV; ++x) {
+      const int at = tid + BS_NT * x, r = at / (BS_DC / 2);
+      const int64_t d = min(d0 + 2 * (at % (BS_DC / 2)), p.D - 2);
+      vq[x] = *(const double2 *)((const double *)p.q + q0 + min(i0 + r, p.nq - 1) * p.q_st + d);
+      vk[x] = *(const double2 *)(kb + min(j0 + r, p.nkb - 1) * p.D + d);
+    }
+  };
+  if constexpr (VEC) fetch(0);
   for (int64_t d0 = 0; d0 < p.D; d0 += BS_DC) {
     const int dn = (int)min((int64_t)BS_DC, p.D - d0);
     __syncthreads();
-    for (int x = tid; x < TQ * BS_DC; x += BS_NT) {
-      const int r = x / BS_DC, dd = x % BS_DC;
-      const int64_t at = q0 + (i0 + r) * p.q_st + d0 + dd;
-      double v = 0.0;
-      if (dd < dn && i0 + r < p.nq) v = F64 ? ((const double *)p.q)[at] : load_as_f64(p.q, at, p.q_dt);
-      sq[dd][r] = v;
-    }
-    for (int x = tid; x < TK * BS_DC; x += BS_NT) {
-      const int r = x / BS_DC, dd = x % BS_DC;
-      sk[dd][r] = (dd < dn && j0 + r < p.nkb) ? kb[(j0 + r) * p.D + d0 + dd] : 0.0;
+    if constexpr (VEC) {
+#pragma unroll
+      for (int x = 0; x < NV; ++x) {
+        const int at = tid + BS_NT * x, r = at / (BS_DC / 2), dd = 2 * (at % (BS_DC / 2));
+        sq[dd][r] = vq[x].x;
+        sq[dd + 1][r] = vq[x].y;
+        sk[dd][r] = vk[x].x;
+        sk[dd + 1][r] = vk[x].y;
+      }
+    } else {
+      for (int x = tid; x < TQ * BS_DC; x += BS_NT) {
+        const int r = x / BS_DC, dd = x % BS_DC;
+        const int64_t at = q0 + (i0 + r) * p.q_st + d0 + dd;
+        double v = 0.0;
+        if (dd < dn && i0 + r < p.nq) v = F64 ? ((const double *)p.q)[at] : load_as_f64(p.q, at, p.q_dt);
+        sq[dd][r] = v;
+      }
+      for (int x = tid; x < TK * BS_DC; x += BS_NT) {
+        const int r = x / BS_DC, dd = x % BS_DC;
+        sk[dd][r] = (dd < dn && j0 + r < p.nkb) ? kb[(j0 + r) * p.D + d0 + dd] : 0.0;
+      }
     }
     __syncthreads();
-    for (int dd = 0; dd < dn; ++dd) {
+    if constexpr (VEC)
+      if (d0 + BS_DC < p.D) fetch(d0 + BS_DC);
+    auto products = [&](int dd) {
       double qv[RQ], kv[RK];
 #pragma unroll
       for (int a = 0; a < RQ; ++a) qv[a] = sq[dd][RQ * tq + a];
 #pragma unroll
-      for (int c = 0; c < RK; ++c) kv[c] = sk[dd][RK * tk + c];
+      for (int c = 0; c < RK; ++c) kv[c] = sk[dd][col(c)];
 #pragma unroll
       for (int a = 0; a < RQ; ++a)
 #pragma unroll
         for (int c = 0; c < RK; ++c) acc[a][c] = add_product(acc[a][c], qv[a], kv[c]);
+    };
+    if (dn == BS_DC) {
+#pragma unroll 8
+      for (int dd = 0; dd < BS_DC; ++dd) products(dd);
+    } else {
+      for (int dd = 0; dd < dn; ++dd) products(dd);
     }
   }
 #pragma unroll
@@ -314,7 +355,7 @@ __global__ __launch_bounds__(BS_NT) void block_score_kernel(ScKP p) {
     if (i >= p.nq) continue;
 #pragma unroll
     for (int c = 0; c < RK; ++c) {
-      const int64_t j = j0 + RK * tk + c;
+      const int64_t j = j0 + col(c);
       if (j < p.nkb) p.scores[(bh * p.nq + i) * p.nkb + j] = acc[a][c];
     }
   }
@@ -343,10 +384,14 @@ static void block_scores(const ScKP &p, int64_t B, hipStream_t st) {
   const dim3 tiles((unsigned)ceil_div(p.nkb, 64), (unsigned)ceil_div(p.nq, 64), (unsigned)(B * p.Hq));
   const bool rows = p.nq >= 16 && p.D % 8 == 0 && p.D <= SC_D && (uintptr_t)p.q % 16 == 0 &&
                     p.q_sb % ev == 0 && p.q_sh % ev == 0 && p.q_st % ev == 0;
-  if (p.q_dt == LA_F64)
-    block_score_kernel<true><<<tiles, BS_NT, 0, st>>>(p);
+  const bool vec = p.D % 2 == 0 && (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.kbar % 16 == 0 &&
+                   p.q_sb % 2 == 0 && p.q_sh % 2 == 0 && p.q_st % 2 == 0;
+  if (p.q_dt == LA_F64 && vec)
+    block_score_kernel<true, true><<<tiles, BS_NT, 0, st>>>(p);
+  else if (p.q_dt == LA_F64)
+    block_score_kernel<true, false><<<tiles, BS_NT, 0, st>>>(p);
   else if (!rows)
-    block_score_kernel<false><<<tiles, BS_NT, 0, st>>>(p);
+    block_score_kernel<false, false><<<tiles, BS_NT, 0, st>>>(p);
   else if (p.q_dt == LA_F32)
     launch_row_scores<LA_F32>(p, B, st);
   else if (p.q_dt == LA_BF16)

@@ -70,3 +70,18 @@ def test_block_lists_place_sinks_and_windows(dev, T, topk, sink, window):
     n = min(ref.shape[-1], ids.shape[-1])
     assert np.array_equal(ids.cpu().numpy()[..., :n], ref[..., :n])
     assert np.array_equal(counts.cpu().numpy(), (ref >= 0).sum(-1))
+
+
+@pytest.mark.parametrize("nb,D", [(1, 2), (63, 30), (64, 32), (65, 34), (130, 66), (66, 33), (70, 160)])
+def test_pooled_scores_in_every_tile_form(dev, nb, D):
+    """Pooled q on 64 x 64 tiles: partial tiles and slices of 32 dims, staged in
+    pairs of dims (even D) or one by one (odd D)."""
+    g = torch.Generator().manual_seed(D)
+    q = torch.randn(2, 4, 4 * nb - 1, D, generator=g).bfloat16()
+    k = torch.randn(2, 2, 4 * nb - 1, D, generator=g).bfloat16()
+    ids, counts = block_select_hip(q.to(dev), k.to(dev), block=4, topk=7, sink_blocks=1, window_blocks=1)
+    ref = oracle.block_select(q, k, block=4, topk=7, sink_blocks=1, window_blocks=1)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    n = min(ref.shape[-1], ids.shape[-1])
+    assert np.array_equal(ids.cpu().numpy()[..., :n], ref[..., :n])
+    assert np.array_equal(counts.cpu().numpy(), (ref >= 0).sum(-1))

@@ -70,6 +70,11 @@ class _Totals:
             self._host = self.totals.tolist()
         return self._host
 
+    def __getstate__(self):
+        # a copied or saved variant holds the numbers, not the device's memory or stream
+        self._read()
+        return {**self.__dict__, "totals": None, "stream": None}
+
     def reads(self) -> float:
         """Mean tokens read per query row."""
         return self._read()[0] / self.rows

@@ -3,6 +3,9 @@ whole numbers, equal to a count over expanded lists."""
 
 from __future__ import annotations
 
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -52,3 +55,12 @@ def test_stats_read_when_asked(dev, name):
     with torch.cuda.stream(torch.cuda.Stream()):
         assert m2.stats() == per_chunk[-1]
     assert all(isinstance(x, float) for x in m2.stats().values())
+
+
+def test_copied_and_saved_variants_keep_their_stats(dev):
+    cfg = AttnConfig(n_heads=4, n_kv_heads=2, head_dim=64, block_size=16, topk_blocks=2)
+    q, k, v = (torch.randn(1, h, 100, 64, device=dev) for h in (4, 2, 2))
+    m = build("hip_moba", cfg)
+    m.forward(q, k, v)
+    assert copy.deepcopy(m).stats() == m.stats()
+    assert pickle.loads(pickle.dumps(m)).stats() == m.stats()

@@ -184,13 +184,15 @@ int la_sparse_attention_noalloc(const la_sparse_attn_args *a, const la_kv *kv, v
 
 /*
  * Totals of list reads, for read accounting (core.py:281-306 reports means of
- * them): totals[0] = the tokens the lists cover, entry u of a row at position
+ * them), as LA_LIST_READS_PARTS pairs whose sums are: first words = the tokens the lists cover, entry u of a row at position
  * offset + t covering the tokens of [u*unit, (u+1)*unit) below
- * min(offset + t + 1, t_k) (-1 entries none); totals[1] = the sum of `counts`
+ * min(offset + t + 1, t_k) (-1 entries none); second words = the sum of `counts`
  * (n_counts of them; NULL: 0).  ids: [B][L][ceil(Tq/rep)][W] at element strides
  * id_sb/id_sh/id_st (0 allowed), each list shared by `rep` consecutive
- * queries.  totals: two device words, written (not added to).
+ * queries.  totals: 2 * LA_LIST_READS_PARTS device words, all written (not added
+ * to).
  */
+#define LA_LIST_READS_PARTS 256
 int la_list_reads(const int32_t *ids, int64_t id_sb, int64_t id_sh, int64_t id_st, int64_t B,
                   int64_t L, int64_t Tq, int64_t W, int64_t rep, int64_t unit, int64_t offset,
                   int64_t t_k, const int32_t *counts, int64_t n_counts, uint64_t *totals,

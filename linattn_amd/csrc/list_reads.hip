@@ -9,18 +9,14 @@ struct LrKP {
   const int32_t *ids, *counts;
   int64_t id_sb, id_sh, id_st, L, Tq, W, rep, unit, offset, t_k, rows, n_counts;
   uint64_t *totals;
-  int32_t add;  // several workgroups: totals are cleared first and added to
-  int32_t lw;   // log2 of the lanes of a row
+  int32_t lw;  // log2 of the lanes of a row
 };
-
-__global__ void list_reads_clear(uint64_t *totals) {
-  if (threadIdx.x < 2) totals[threadIdx.x] = 0;
-}
 
 // 2^lw lanes per row (at least its entries, at most a wave); the same totals as
 // torch's masks and sums over the expanded lists, which took ten launches and two
-// host reads per call: 150 us of a 256-query chunk, about 7 us and no host read
-// here.
+// host reads per call: 150 us of a 256-query chunk, about 6 us and no host read
+// here.  Every workgroup writes a pair of its own, and the first one zeros the
+// pairs past the grid: sums in one pair took a launch of 3.7 us that cleared it.
 __global__ __launch_bounds__(256) void list_reads_kernel(LrKP p) {
   __shared__ uint64_t part[2][4];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -65,11 +61,10 @@ __global__ __launch_bounds__(256) void list_reads_kernel(LrKP p) {
   __syncthreads();
   if (threadIdx.x < 2) {
     const uint64_t s = part[threadIdx.x][0] + part[threadIdx.x][1] + part[threadIdx.x][2] + part[threadIdx.x][3];
-    if (p.add)
-      __hip_atomic_fetch_add(p.totals + threadIdx.x, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else
-      p.totals[threadIdx.x] = s;
+    p.totals[2 * blockIdx.x + threadIdx.x] = s;
   }
+  if (blockIdx.x == 0)
+    for (int i = 2 * gridDim.x + threadIdx.x; i < 2 * LA_LIST_READS_PARTS; i += 256) p.totals[i] = 0;
 }
 
 }  // namespace la
@@ -85,20 +80,12 @@ extern "C" int la_list_reads(const int32_t *ids, int64_t id_sb, int64_t id_sh, i
   const int64_t rows = B * L * Tq;
   LA_REQUIRE(rows < ((int64_t)1 << 31) && rep < ((int64_t)1 << 31), "la_list_reads: 2^31 rows or more");
   LA_REQUIRE(n_counts >= 0 && (counts || n_counts == 0), "la_list_reads: counts");
-  LrKP p{ids, counts, id_sb, id_sh, id_st, L, Tq, W, rep, unit, offset, t_k, rows, n_counts, totals, 0, 0};
+  LrKP p{ids, counts, id_sb, id_sh, id_st, L, Tq, W, rep, unit, offset, t_k, rows, n_counts, totals, 0};
   p.lw = std::min(6, ilog2(W));
-  // One workgroup while it has few rows to read (a second launch costs more);
-  // else as many as give a thread its rows at a time, at most 256: each adds to
-  // the same two words (1024 of them took 15 us, the adds alone).
+  // As many workgroups as give a thread its rows at a time.
   const int64_t turns = ceil_div(rows, 256 >> p.lw) * ceil_div(W, (int64_t)1 << p.lw);
-  const unsigned grid = turns <= 8 ? 1u : (unsigned)std::min<int64_t>(256, ceil_div(turns, 8));
-  hipStream_t st = (hipStream_t)stream;
-  p.add = grid > 1;
-  if (p.add) {
-    list_reads_clear<<<dim3(1), 64, 0, st>>>(totals);
-    LA_LAUNCHED();
-  }
-  list_reads_kernel<<<dim3(grid), 256, 0, st>>>(p);
+  const unsigned grid = (unsigned)std::min<int64_t>(LA_LIST_READS_PARTS, ceil_div(turns, 8));
+  list_reads_kernel<<<dim3(grid), 256, 0, (hipStream_t)stream>>>(p);
   LA_LAUNCHED();
   return LA_OK;
 }

@@ -54,7 +54,7 @@ class _Totals:
         if ids.stride(3) != 1:
             ids = ids.contiguous()
             sb, sh, st = ids.stride(0), ids.stride(1), ids.stride(2)
-        self.totals = torch.empty(2, dtype=torch.int64, device=ids.device)
+        self.totals = torch.empty(N.LIST_READS_PARTS, 2, dtype=torch.int64, device=ids.device)
         self.stream = torch.cuda.current_stream(ids.device)
         self.rows = B * L * t_q
         self.lists = counts.numel() if counts is not None else 0
@@ -67,7 +67,7 @@ class _Totals:
     def _read(self):
         if self._host is None:
             self.stream.synchronize()
-            self._host = self.totals.tolist()
+            self._host = self.totals.cpu().sum(0).tolist()
         return self._host
 
     def __getstate__(self):

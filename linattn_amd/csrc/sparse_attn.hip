@@ -931,12 +931,37 @@ __global__ __launch_bounds__(QD_NT, 4) void quest_decode_fused_kernel(QsKP a, At
   finish_row<G, 128, QD_NW>(p, rc, row, 0, L.u.att.acc, L.u.att.m, L.u.att.l);
 }
 
-// Merge the split partials of the (row, head)s: 32 lanes each, eight per
-// workgroup, a lane D / 32 neighbouring dims.  Latency-bound, so four splits'
-// maxima, sums and values are read at once: one memory round trip (a merge of
-// 32768 rows of two parts took 27 us with one workgroup per row and a round
-// trip per split, 9 us like this).  TILES: the parts of list_tile.hip, whose
-// left-out tiles hold none and whose results are marked where not finite.
+// Merge the split partials of a (row, head): one workgroup, a thread per dim.
+// Bound by the latency of its loads (the maxima, then a value per split), so at
+// few rows it is the spread over the CUs and not the loads per thread that
+// counts: see launch_merge.
+template <int D>
+__global__ __launch_bounds__(D) void sparse_attn_combine_row(AttnKP p, int64_t G) {
+  const int64_t rg = blockIdx.x;
+  const int64_t r = rg / G, g = rg % G;
+  const int64_t t = r % p.Tq;
+  const int64_t ih = (r / p.Tq) % p.ids_heads;
+  const int64_t b = r / (p.Tq * p.ids_heads);
+  const int64_t h = ((p.ids_heads == p.Hkv) ? ih * G : ih) + g;
+  const float *ml = p.ws_ml + rg * p.splits * 2;
+  const int d = threadIdx.x;
+  float M = __int_as_float(0xff800000);
+  for (int64_t s = 0; s < p.splits; ++s) M = fmaxf(M, ml[2 * s]);
+  const float Mu = (M == __int_as_float(0xff800000)) ? 0.f : M;
+  float L = 0.f, A = 0.f;
+  for (int64_t s = 0; s < p.splits; ++s) {
+    const float sc = fast_exp2(ml[2 * s] - Mu);
+    L += ml[2 * s + 1] * sc;
+    A += p.ws_acc[(rg * p.splits + s) * D + d] * sc;
+  }
+  const float o = L > 0.f ? A / L : 0.f;
+  store_from_f32(p.out, b * p.o_sb + h * p.o_sh + t * p.o_st + d, p.out_dt, o);
+}
+
+// The same for many (row, head)s: 32 lanes each, eight per workgroup, a lane
+// D / 32 neighbouring dims, four splits' maxima, sums and values read at once (one
+// memory round trip).  TILES: the parts of list_tile.hip, whose left-out tiles
+// hold none and whose results are marked where not finite.
 template <int D, bool TILES>
 __global__ __launch_bounds__(256) void sparse_attn_combine(AttnKP p, int64_t G, int64_t RG,
                                                            ListTileGate gt) {
@@ -1026,6 +1051,24 @@ constexpr int unroll_for(int D) {
   return 4;
 }
 
+// A workgroup per (row, head) up to MERGE_ROWS of them (decode), eight rows a
+// workgroup above: at fewer rows eight to a workgroup leave CUs idle, at more the
+// launch of a workgroup per row is what takes the time.  D = 128, one / eight rows
+// a workgroup, us: 128 (row, head)s of 4 splits 3.9 / 4.5, of 16 7.0 / 8.4; 512 of
+// 8 4.8 / 5.7; 2048 of 2 4.2 / 5.1, of 16 9.2 / 9.6; 4096 of 2 5.4 / 5.3, of 4 6.2
+// / 5.3; 8192 of 2 9.0 / 5.5; 32768 of 2 27.5 / 11.2.
+constexpr int64_t MERGE_ROWS = 2048;
+template <int D>
+static int launch_merge(const AttnKP &p, int64_t G, hipStream_t st) {
+  const int64_t RG = p.B * p.ids_heads * p.Tq * G;
+  if (RG <= MERGE_ROWS)
+    sparse_attn_combine_row<D><<<dim3((unsigned)RG), D, 0, st>>>(p, G);
+  else
+    sparse_attn_combine<D, false><<<dim3((unsigned)ceil_div(RG, 8)), 256, 0, st>>>(p, G, RG, ListTileGate{});
+  LA_LAUNCHED();
+  return LA_OK;
+}
+
 template <int KT, int D, int G, bool PAGED>
 static int launch_attn(const AttnKP &p, hipStream_t st) {
   constexpr int UNR = unroll_for<KT>(D);
@@ -1039,11 +1082,7 @@ static int launch_attn(const AttnKP &p, hipStream_t st) {
   else
     sparse_attn_kernel<KT, D, G, UNR, PAGED><<<grid, SA_NT, 0, st>>>(p);
   LA_LAUNCHED();
-  if (p.splits > 1) {
-    const int64_t RG = p.B * p.ids_heads * p.Tq * G;
-    sparse_attn_combine<D, false><<<dim3((unsigned)ceil_div(RG, 8)), 256, 0, st>>>(p, G, RG, ListTileGate{});
-    LA_LAUNCHED();
-  }
+  if (p.splits > 1) return launch_merge<D>(p, G, st);
   return LA_OK;
 }
 

@@ -268,18 +268,22 @@ __global__ __launch_bounds__(256) void few_row_score_kernel(ScKP p) {
 // on 128 dims, causal: 203 us loaded one by one, 157 loaded ahead, 144 with columns
 // read in runs of 256 bytes and whole slices unrolled (56 for the instructions; held
 // to 128 registers for a fourth workgroup per CU it spills and takes 168).
+// TQ = 4: one score per thread, for up to four rows a head, of which a 64-row tile
+// would stage and multiply 60 empty ones.  Gate calls of 64 heads on 4 KV heads, one
+// query, 256 blocks, batch 8: 61 us on 64-row tiles, 30 here; 16 heads, four queries,
+// D = 192, batch 4: 34 and 20.
 constexpr int BS_DC = 32, BS_NT = 256;
-template <bool F64, bool VEC>
+template <bool F64, bool VEC, int TQ = 64>
 __global__ __launch_bounds__(BS_NT) void block_score_kernel(ScKP p) {
-  constexpr int TQ = 64, RQ = 4, RK = 4, TX = BS_NT / (TQ / RQ), TK = TX * RK;
+  constexpr int RQ = TQ == 64 ? 4 : 1, RK = RQ, TX = BS_NT / (TQ / RQ), TK = TX * RK;
   constexpr int NV = TQ * BS_DC / (2 * BS_NT);  // pairs of a thread's share of a slice
-  static_assert(TQ == TK && (!VEC || F64), "");
+  static_assert(TK == 64 && (TQ == 64 || TQ == 4) && (!VEC || (F64 && TQ == TK)), "");
   __shared__ __align__(16) double sq[BS_DC][TQ + 2];
   __shared__ __align__(16) double sk[BS_DC][TK + 2];
   const int tid = threadIdx.x;
   // rows RQ*tq.., columns 2*tk, 2*tk + 1 and TK/2 on: 16 threads read 256 bytes in a row
   const int tq = tid / TX, tk = tid % TX;
-  auto col = [&](int c) { return (c >> 1) * (TK / 2) + 2 * tk + (c & 1); };
+  auto col = [&](int c) { return RK == 1 ? tk : (c >> 1) * (TK / 2) + 2 * tk + (c & 1); };
   const int64_t i0 = (int64_t)blockIdx.y * TQ, j0 = (int64_t)blockIdx.x * TK;
   const int64_t bh = blockIdx.z;
   const int64_t b = bh / p.Hq, h = bh % p.Hq;
@@ -291,7 +295,7 @@ __global__ __launch_bounds__(BS_NT) void block_score_kernel(ScKP p) {
   for (int a = 0; a < RQ; ++a)
 #pragma unroll
     for (int c = 0; c < RK; ++c) acc[a][c] = 0.0;
-  double2 vq[NV], vk[NV];
+  double2 vq[VEC ? NV : 1], vk[VEC ? NV : 1];
   // (rows and dims past the end read the last ones; their sums are not stored or not formed)
   auto fetch = [&](int64_t d0) {
 #pragma unroll
@@ -373,8 +377,9 @@ static void launch_row_scores(const ScKP &p, int64_t B, hipStream_t st) {
 }
 
 // Scores of every row and column of (B * Hq) heads.  Up to SF_ROWS rows per KV
-// head take the decode form; the row form needs q rows in 16-byte pieces, and
-// below 16 rows its lanes are mostly idle.
+// head of up to SF_D dims take the decode form that reads the means once for all of
+// them, other calls of up to four rows per head the 4-row tiles; the row form needs
+// q rows in 16-byte pieces, and below 16 rows its lanes are mostly idle.
 static void block_scores(const ScKP &p, int64_t B, hipStream_t st) {
   const int64_t ev = p.q_dt == LA_F32 ? 4 : 8;
   if (p.Hq / p.Hkv * p.nq <= SF_ROWS && p.D <= SF_D && p.D % 2 == 0 && (uintptr_t)p.kbar % 16 == 0) {
@@ -386,7 +391,12 @@ static void block_scores(const ScKP &p, int64_t B, hipStream_t st) {
                     p.q_sb % ev == 0 && p.q_sh % ev == 0 && p.q_st % ev == 0;
   const bool vec = p.D % 2 == 0 && (uintptr_t)p.q % 16 == 0 && (uintptr_t)p.kbar % 16 == 0 &&
                    p.q_sb % 2 == 0 && p.q_sh % 2 == 0 && p.q_st % 2 == 0;
-  if (p.q_dt == LA_F64 && vec)
+  const dim3 few(tiles.x, 1, tiles.z);
+  if (p.nq <= 4 && p.q_dt == LA_F64)
+    block_score_kernel<true, false, 4><<<few, BS_NT, 0, st>>>(p);
+  else if (p.nq <= 4)
+    block_score_kernel<false, false, 4><<<few, BS_NT, 0, st>>>(p);
+  else if (p.q_dt == LA_F64 && vec)
     block_score_kernel<true, true><<<tiles, BS_NT, 0, st>>>(p);
   else if (p.q_dt == LA_F64)
     block_score_kernel<true, false><<<tiles, BS_NT, 0, st>>>(p);

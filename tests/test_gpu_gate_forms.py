@@ -20,6 +20,11 @@ pytestmark = pytest.mark.gpu
     (8, 2, 2, 65, 128, torch.float32),
     (4, 4, 8, 64, 64, torch.float16),
     (4, 4, 9, 33, 64, torch.float16),      # one row more than the decode form takes
+    (32, 2, 1, 65, 128, torch.bfloat16),   # 4-row tiles: groups the decode form has no room for
+    (16, 2, 4, 64, 128, torch.float32),
+    (16, 2, 5, 64, 128, torch.float32),    # one row more than those take
+    (4, 4, 1, 63, 192, torch.bfloat16),    # dims it has no room for
+    (4, 2, 3, 66, 33, torch.float16),
     (8, 2, 15, 31, 64, torch.bfloat16),    # tiles: too few rows
     (4, 2, 16, 33, 128, torch.bfloat16),   # rows: the fewest, a column past a group
     (2, 1, 64, 32, 72, torch.bfloat16),

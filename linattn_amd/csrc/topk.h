@@ -38,7 +38,6 @@ struct TopkKParams {
   // shorter sequence: nothing selected, no sink, no own unit)
   const int32_t *b_lens;
   int64_t rows_per_b, b_len_unit;
-  int32_t row32;  // tk_row_fits_32 (set by topk_launch)
 };
 
 // The row (group) a workgroup selects for, its valid prefix and forced unit.
@@ -88,12 +87,6 @@ __device__ __forceinline__ TkRow tk_row(const TopkKParams &p, int64_t gi) {
   r.force = p.force_own && own >= 0 && own < r.n_v;
   r.K = min(p.k, r.n_v);
   return r;
-}
-
-// tk_row in the arithmetic the launch chose (64-bit quotients cost a wave of a
-// short row more than its selection does).
-__device__ __forceinline__ TkRow tk_row_of(const TopkKParams &p, int64_t gi) {
-  return p.row32 ? tk_row<true>(p, gi) : tk_row<false>(p, gi);
 }
 
 // Whether tk_row<true> is exact for every group of p: the dividends (group

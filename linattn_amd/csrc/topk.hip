@@ -170,6 +170,19 @@ __device__ void tk_select(const RowKeys &key, int64_t n_v, int64_t K, TkShared &
   __syncthreads();
 }
 
+// What these kernels take on top.  (Not a member of TopkKParams: the radix kernels
+// hold that one among their parameters, and with eight bytes more in it the compiler
+// loads those in more and smaller pieces: 7.6 -> 8.2 us a stage.)
+struct TopkRowKP : TopkKParams {
+  int32_t row32;  // tk_row_fits_32
+};
+
+// tk_row in the arithmetic the launch chose (64-bit quotients cost a wave of a
+// short row more than its selection does).
+__device__ __forceinline__ TkRow tk_row_of(const TopkRowKP &p, int64_t gi) {
+  return p.row32 ? tk_row<true>(p, gi) : tk_row<false>(p, gi);
+}
+
 // the candidate row of a segmented top-k's final level (G = 1), or null
 __device__ __forceinline__ const int32_t *tk_cand_row(const TopkKParams &p, const TkRow &rw) {
   return p.cand_idx ? p.cand_idx + ((rw.br - rw.tl) * p.G + rw.tl) * p.row_stride + rw.seg0
@@ -182,7 +195,7 @@ __device__ __forceinline__ void tk_emit_bitmap(const TopkKParams &p, uint32_t *b
                      p.out_count ? p.out_count + rw.orow : nullptr, wtmp, tk_cand_row(p, rw));
 }
 
-__global__ __launch_bounds__(TK_NT) void topk_rows_kernel(TopkKParams p) {
+__global__ __launch_bounds__(TK_NT) void topk_rows_kernel(TopkRowKP p) {
   extern __shared__ __align__(16) unsigned char dyn[];
   __shared__ TkShared sh;
   const int tid = threadIdx.x;
@@ -414,7 +427,7 @@ __device__ __forceinline__ void tk_bitonic_desc(uint64_t (&c)[E], int tid, uint6
 // so every further resident workgroup per CU pays (the whole C2 indexer call
 // took 0.767 ms with two per CU, 0.630 with three, 0.609 with four).
 template <int KPT, int E, bool BITMAP>
-__global__ __launch_bounds__(TK_NT, (!BITMAP && KPT >= 32) ? 4 : 1) void topk_reg_kernel(TopkKParams p) {
+__global__ __launch_bounds__(TK_NT, (!BITMAP && KPT >= 32) ? 4 : 1) void topk_reg_kernel(TopkRowKP p) {
   constexpr int P = TK_NT * E;  // sort width (sorted form)
   extern __shared__ __align__(16) unsigned char dyn[];
   __shared__ TkRegShared<KPT> sr;
@@ -838,7 +851,7 @@ __global__ __launch_bounds__(TK_NT, (!BITMAP && KPT >= 32) ? 4 : 1) void topk_re
 // (with the row arithmetic in 32 bits, 32768 rows of 64 units: 33 -> 22 us; of at
 // most 512 units: 70 -> 55 us).
 template <int KPL, bool ONE>
-__global__ __launch_bounds__(TK_NT) void topk_wave_kernel(TopkKParams p) {
+__global__ __launch_bounds__(TK_NT) void topk_wave_kernel(TopkRowKP p) {
   constexpr int WORDS = 2 * KPL;  // 32-bit bitmap words per row
   __shared__ uint32_t bms[ONE ? 1 : TK_NW][WORDS];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1012,7 +1025,7 @@ int topk_launch_ws(TopkKParams p, void *ws, int64_t ws_bytes, hipStream_t st) {
 }
 
 template <bool BITMAP, int KPT>
-static int launch_reg_e(const TopkKParams &p, int E, size_t bytes, hipStream_t st) {
+static int launch_reg_e(const TopkRowKP &p, int E, size_t bytes, hipStream_t st) {
   const dim3 grid((unsigned)p.NG);
   if constexpr (BITMAP) {
     topk_reg_kernel<KPT, 1, true><<<grid, TK_NT, bytes, st>>>(p);
@@ -1033,7 +1046,7 @@ static int launch_reg_e(const TopkKParams &p, int E, size_t bytes, hipStream_t s
 // Register-resident form: rows of at most 8192 keys (16384 for the bitmap
 // form; a segment's length in segmented mode); sorted output for k up to 4096
 // of one row per group.
-static int launch_reg(const TopkKParams &p, hipStream_t st) {
+static int launch_reg(const TopkRowKP &p, hipStream_t st) {
   int kpt = 1;
   while (kpt * TK_NT < p.n_lds) kpt <<= 1;
   const int64_t kk = std::min(p.k, p.n_lds);
@@ -1062,7 +1075,7 @@ static int launch_reg(const TopkKParams &p, hipStream_t st) {
 }
 
 template <bool ONE>
-static void launch_wave(const TopkKParams &p, int kpl, dim3 grid, hipStream_t st) {
+static void launch_wave(const TopkRowKP &p, int kpl, dim3 grid, hipStream_t st) {
   switch (kpl) {
     case 1: topk_wave_kernel<1, ONE><<<grid, TK_NT, 0, st>>>(p); break;
     case 2: topk_wave_kernel<2, ONE><<<grid, TK_NT, 0, st>>>(p); break;
@@ -1072,9 +1085,9 @@ static void launch_wave(const TopkKParams &p, int kpl, dim3 grid, hipStream_t st
   }
 }
 
-int topk_launch(TopkKParams p, hipStream_t st) {
-  if (p.NG <= 0) return LA_OK;
-  p.row32 = tk_row_fits_32(p) ? 1 : 0;
+int topk_launch(TopkKParams params, hipStream_t st) {
+  if (params.NG <= 0) return LA_OK;
+  TopkRowKP p{params, tk_row_fits_32(params) ? 1 : 0};
   p.use_bitmap = (p.G > 1 || p.sink > 0 || p.window > 0 || p.order == 1) ? 1 : 0;
   p.n_lds = p.seg_len > 0 ? std::min(p.seg_len, p.n) : p.n;
   p.bitmap_words = (p.n_lds + 31) / 32;

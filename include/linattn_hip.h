@@ -271,7 +271,9 @@ int la_quest_select(const la_quest_select_args *a, void *stream);
  * la_quest_scores followed by la_topk_rows with group = 1, order = 0, force_own =
  * 1, pos_unit = page_size.  Returns LA_ERR_UNSUPPORTED (nothing launched) when
  * the metadata is not page-minor (m_sp == 1), for more than 1024 pages or for
- * k > 256; callers then use the two separate entry points.
+ * k > 256, and from 2^26 rows on (2^24 for more than 256 pages); callers then use
+ * the two separate entry points, which are also the faster ones for k > 128 and for
+ * many rows over more than 256 pages.
  */
 int la_quest_select_heads(const la_quest_select_args *a, void *stream);
 

@@ -628,10 +628,11 @@ extern "C" int la_quest_select_heads(const la_quest_select_args *a, void *stream
   const int rc = validate_select(a);
   if (rc != LA_OK) return rc;
   const int64_t rows = a->B * a->Hq * a->Tq;
-  // page-minor metadata (any alignment); rows that one workgroup's LDS holds
+  // page-minor metadata (any alignment); rows that one workgroup's LDS holds; fewer
+  // than 2^32 threads (four rows or one per workgroup)
   const int64_t G = a->Hq / a->Hkv;
-  if (a->m_sp != 1 || a->n_pages > 1024 || rows >= ((int64_t)1 << 31) || std::min(a->k, a->n_pages) > 256 ||
-      !(G == 1 || G == 2 || G == 4 || G == 8))
+  if (a->m_sp != 1 || a->n_pages > 1024 || rows >= ((int64_t)1 << (a->n_pages <= 256 ? 26 : 24)) ||
+      std::min(a->k, a->n_pages) > 256 || !(G == 1 || G == 2 || G == 4 || G == 8))
     return fail(LA_ERR_UNSUPPORTED, "la_quest_select_heads: shape or metadata layout not fused");
   QsKP k = select_params(a);
   k.width = k.k;

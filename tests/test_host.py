@@ -86,3 +86,20 @@ def test_backend_report():
 def test_page_meta_is_page_minor():
     mn, mx = alloc_page_meta(2, 3, 10, 64, torch.bfloat16, "cpu")
     assert mn.shape == (2, 3, 10, 64) and mn.stride(2) == 1 and mn.stride(3) == 12
+
+
+def test_head_selection_refuses_what_its_grid_cannot_hold():
+    """Before any launch: one row a workgroup (more than 256 pages) or four, fewer than
+    2^32 threads."""
+    import ctypes
+
+    from linattn_amd import _native as N
+    for rows, pages in ((1 << 26, 64), (1 << 24, 257)):
+        a = N.LaQuestSelectArgs()
+        a.q = a.page_min = a.page_max = a.out_idx = 4096  # (never read)
+        a.B, a.Hq, a.Hkv, a.Tq, a.D = 1, 1, 1, rows, 64
+        a.q_sb = a.q_sh = a.q_st = 64
+        a.n_pages, a.page_size, a.k, a.pos_offset = pages, 16, 4, 0
+        a.m_sb, a.m_sh, a.m_sp, a.m_sd = 64 * pages, 64 * pages, 1, pages
+        a.q_dtype = a.meta_dtype = N.LA_F32
+        assert N.load().la_quest_select_heads(ctypes.byref(a), None) == N.LA_ERR_UNSUPPORTED

@@ -139,6 +139,27 @@ def _topk(scores: torch.Tensor, *, k: int, width: int, group: int, order: int,
     return ids, counts, vals
 
 
+def _heads_in_one_kernel(rows: int, P: int, k: int, D: int, G: int) -> bool:
+    """Whether ``la_quest_select_heads`` is faster than scores and top-k in two launches.
+
+    It reads the bounds (half of them) per query head and not per KV head, a row at a
+    time, and one wave ranks a row's kept pages by k^2 / 64 compares.  Whole calls, two
+    launches / one kernel, us, bf16 unless said.  k <= 32, at most 256 pages: one kernel
+    throughout (8 rows 1.2-1.5 times faster, 16384 rows 1.5).  k = 32, more pages: D =
+    128, 512 pages, 64 rows 27 / 22, 2048 rows 64 / 68, 16384 rows 388 / 448 (with four
+    heads a KV head 312 / 448); 1024 pages, 512 rows 36 / 38 (four heads 45 / 38); D =
+    64, 16384 rows, 512 pages, one head 284 / 246, 2048 rows, 1024 pages 69 / 49, with
+    four heads 71 / 87.  k = 128, D = 128, 256 pages: 512 rows 29 / 32, 2048 rows 47 /
+    39, four heads, 512 rows 41 / 33.  k = 256, 256 pages, 8 rows: 22 / 44."""
+    if k > 128 or P > 1024:
+        return False
+    if P <= 256:
+        return k <= 64 or D <= 64 or G > 1 or rows >= 2048
+    if k <= 64 and G == 1 and D <= 64:
+        return True
+    return (k <= 64 or G > 1) and rows <= (256 if G == 1 and P > 512 else 512)
+
+
 def quest_select_hip(q: torch.Tensor, mins: torch.Tensor, maxs: torch.Tensor, *, page_size: int,
                      topk: int, offset: int = 0, gqa_union: bool = True,
                      positions: Optional[torch.Tensor] = None
@@ -163,9 +184,11 @@ def quest_select_hip(q: torch.Tensor, mins: torch.Tensor, maxs: torch.Tensor, *,
     if positions is not None and (positions.dtype != torch.int32 or positions.shape != (B,)
                                   or not positions.is_contiguous()):
         raise ValueError("positions must be contiguous int32 (B,)")
-    if mins.stride() == maxs.stride() and mins.dtype == maxs.dtype:
+    union = gqa_union and G > 1
+    # (with a position per sequence, two launches would be two per sequence)
+    if mins.stride() == maxs.stride() and mins.dtype == maxs.dtype and (
+            union or positions is not None or _heads_in_one_kernel(B * Hq * Tq, P, k, D, G)):
         # one pass: scores and top-k per head, and the union of a group's heads
-        union = gqa_union and G > 1
         heads, width = (Hkv, G * k) if union else (Hq, k)
         ids = torch.empty(B, heads, Tq, width, dtype=torch.int32, device=dev)
         counts = torch.empty(B, heads, Tq, dtype=torch.int32, device=dev)

@@ -31,6 +31,14 @@ def _two_launches(q, mins, maxs, *, page_size, topk, offset):
     (1, 8, 8, 5, 257, 128, 33, torch.float32),
     (2, 2, 2, 2, 512, 64, 200, torch.bfloat16),
     (1, 2, 2, 1, 1000, 200, 256, torch.float32),
+    # both sides of where two launches take over: rows, k, dims, heads a KV head
+    (1, 8, 8, 64, 257, 128, 9, torch.bfloat16),
+    (1, 9, 9, 57, 257, 128, 9, torch.bfloat16),
+    (1, 4, 4, 600, 300, 64, 64, torch.float32),
+    (1, 4, 2, 5, 300, 64, 128, torch.float32),
+    (1, 4, 2, 5, 300, 64, 129, torch.float32),
+    (1, 2, 2, 3, 256, 128, 65, torch.bfloat16),
+    (1, 2, 2, 1100, 256, 128, 65, torch.bfloat16),
 ])
 def test_lists_match_oracle(dev, B, hq, hkv, Tq, pages, D, topk, dtype):
     ps = 4
@@ -66,14 +74,17 @@ def test_ties_and_special_values_rank_as_in_two_launches(dev):
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
 
 
-def test_ragged_positions_equal_one_call_per_sequence(dev):
+@pytest.mark.parametrize("page,topk", [(8, 12), (4, 200), (2, 256), (1, 256)])
+def test_ragged_positions_equal_one_call_per_sequence(dev, page, topk):
+    """(One kernel for every k and row count it has room for: the other form takes a
+    call per sequence.)"""
     g = torch.Generator().manual_seed(1)
     q = torch.randn(3, 4, 1, 64, generator=g).to(dev)
     k = torch.randn(3, 4, 900, 64, generator=g).to(dev)
-    mins, maxs = page_update_hip(k, 8)
+    mins, maxs = page_update_hip(k, page)
     pos = torch.tensor([0, 433, 899], dtype=torch.int32, device=dev)
-    ids, counts = quest_select_hip(q, mins, maxs, page_size=8, topk=12, gqa_union=False, positions=pos)
+    ids, counts = quest_select_hip(q, mins, maxs, page_size=page, topk=topk, gqa_union=False, positions=pos)
     for b in range(3):
-        one, n = quest_select_hip(q[b:b + 1], mins[b:b + 1], maxs[b:b + 1], page_size=8, topk=12,
-                                  gqa_union=False, offset=int(pos[b]))
+        one, n = _two_launches(q[b:b + 1], mins[b:b + 1], maxs[b:b + 1], page_size=page, topk=topk,
+                               offset=int(pos[b]))
         assert torch.equal(ids[b:b + 1], one) and torch.equal(counts[b:b + 1], n)

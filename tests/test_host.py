@@ -103,3 +103,15 @@ def test_head_selection_refuses_what_its_grid_cannot_hold():
         a.m_sb, a.m_sh, a.m_sp, a.m_sd = 64 * pages, 64 * pages, 1, pages
         a.q_dtype = a.meta_dtype = N.LA_F32
         assert N.load().la_quest_select_heads(ctypes.byref(a), None) == N.LA_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("rows,pages,k,D,G,one", [
+    (8, 256, 128, 64, 1, True), (8, 256, 129, 64, 1, False),        # the k^2 ranking
+    (2047, 256, 65, 128, 1, False), (2048, 256, 65, 128, 1, True),
+    (512, 512, 32, 128, 1, True), (513, 512, 32, 128, 1, False),    # the bounds read per row
+    (257, 513, 32, 128, 1, False), (512, 1024, 32, 128, 4, True), (513, 257, 4, 64, 4, False),
+    (1 << 20, 1024, 4, 64, 1, True), (8, 1025, 4, 64, 1, False),
+])
+def test_head_selection_takes_the_faster_form(rows, pages, k, D, G, one):
+    from linattn_amd.kernels.quest_pages import _heads_in_one_kernel
+    assert _heads_in_one_kernel(rows, pages, k, D, G) is one

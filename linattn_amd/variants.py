@@ -42,7 +42,11 @@ __all__ = ["HipAttention", "HipQuest", "HipDSA", "HipMoBA", "HipXAttention", "Hi
 
 class _Totals:
     """Token reads and counts of one selection, summed on the device
-    (``la_list_reads``) with no host read until a mean is asked for."""
+    (``la_list_reads``) with no host read until a mean is asked for.
+
+    Captured into a graph, every replay sums again, on whatever stream it is
+    replayed: the means are then read off the device each time they are asked for,
+    after all of its work."""
 
     def __init__(self, ids: torch.Tensor, unit: int, offset: int, t_q: int, t_k: int,
                  counts: Optional[torch.Tensor] = None, rep: int = 1):
@@ -56,6 +60,7 @@ class _Totals:
             sb, sh, st = ids.stride(0), ids.stride(1), ids.stride(2)
         self.totals = torch.empty(N.LIST_READS_PARTS, 2, dtype=torch.int64, device=ids.device)
         self.stream = torch.cuda.current_stream(ids.device)
+        self.captured = torch.cuda.is_current_stream_capturing()
         self.rows = B * L * t_q
         self.lists = counts.numel() if counts is not None else 0
         self._host = None
@@ -65,15 +70,21 @@ class _Totals:
             "read totals")
 
     def _read(self):
-        if self._host is None:
+        if self._host is not None:
+            return self._host
+        if self.captured:
+            torch.cuda.synchronize(self.totals.device)
+        else:
             self.stream.synchronize()
-            self._host = self.totals.cpu().sum(0).tolist()
-        return self._host
+        sums = self.totals.cpu().sum(0).tolist()
+        if not self.captured:
+            self._host = sums
+        return sums
 
     def __getstate__(self):
         # a copied or saved variant holds the numbers, not the device's memory or stream
-        self._read()
-        return {**self.__dict__, "totals": None, "stream": None}
+        return {**self.__dict__, "_host": self._read(), "totals": None, "stream": None,
+                "captured": False}
 
     def reads(self) -> float:
         """Mean tokens read per query row."""

@@ -64,3 +64,38 @@ def test_copied_and_saved_variants_keep_their_stats(dev):
     m.forward(q, k, v)
     assert copy.deepcopy(m).stats() == m.stats()
     assert pickle.loads(pickle.dumps(m)).stats() == m.stats()
+
+
+@pytest.mark.parametrize("name", ["hip_quest", "hip_moba", "hip_xattention"])
+def test_stats_follow_graph_replays(dev, name):
+    """Each replay's stats are those of its own inputs, also after stats were read
+    before; a copy keeps the numbers it was made with.  (Threshold lists: how many
+    blocks a query keeps depends on the values.)"""
+    cfg = AttnConfig(n_heads=4, n_kv_heads=2, head_dim=64, block_size=16, topk_blocks=2)
+    g = torch.Generator().manual_seed(2)
+    ins = [[torch.randn(1, h, 160, 64, generator=g) * s for h in (4, 2, 2)] for s in (0.1, 1.0, 6.0)]
+    eager, want = build(name, cfg), []
+    for x in ins:
+        out, _ = eager.forward(*(t.to(dev) for t in x))
+        want.append((out, eager.stats()))
+    if name == "hip_xattention":
+        assert len({w["blocks_per_query"] for _, w in want}) == len(ins)
+    m = build(name, cfg)
+    q, k, v = (t.to(dev) for t in ins[0])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        m.forward(q, k, v)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, _ = m.forward(q, k, v)
+    copies = []
+    for i in (0, 1, 2, 0, 2):
+        for t, x in zip((q, k, v), ins[i]):
+            t.copy_(x)
+        graph.replay()
+        assert m.stats() == want[i][1]
+        assert torch.equal(out, want[i][0])
+        copies.append((i, copy.deepcopy(m)))
+    assert all(c.stats() == want[i][1] for i, c in copies)

@@ -32,8 +32,9 @@ struct ListTileGate {
   const int32_t *nlist;  // [b][ngrp][ntile]
   int64_t m_sb, m_sh, m_st;
   int32_t qt, ntile, ngrp, gt;
+  // (h and t below 2^31)
   __device__ __forceinline__ bool tile_left(int64_t b, int64_t h, int64_t t) const {
-    return nlist[(b * ngrp + h / gt) * ntile + t / qt] < 0;
+    return nlist[(b * ngrp + (uint32_t)h / (uint32_t)gt) * ntile + (uint32_t)t / (uint32_t)qt] < 0;
   }
 };
 

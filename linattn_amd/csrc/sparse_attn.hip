@@ -111,9 +111,9 @@ struct RowCtx {
 // caller synchronises before reading the staged entries.
 template <int G, bool PAGED>
 __device__ __forceinline__ RowCtx stage_row(const AttnKP &p, int64_t r, int64_t split,
-                                            int32_t *s_tok0, int32_t *s_phys) {
+                                            int32_t *s_tok0, int32_t *s_phys,
+                                            const int tid = threadIdx.x) {
   RowCtx rc;
-  const int tid = threadIdx.x;
   rc.t = r % p.Tq;
   const int64_t ih = (r / p.Tq) % p.ids_heads;
   rc.b = r / (p.Tq * p.ids_heads);
@@ -448,7 +448,7 @@ struct MfmaLds {
 template <int KT, int G, bool PAGED, bool U16, int NW>
 __device__ __forceinline__ void mfma_attend(const AttnKP &p, const RowCtx &rc,
                                             const int32_t *s_tok0, const int32_t *s_phys,
-                                            MfmaLds<KT, G, NW> &L) {
+                                            MfmaLds<KT, G, NW> &L, const int tid = threadIdx.x) {
   constexpr bool F8 = KT == LA_FP8_E4M3;
   constexpr int ESZ = F8 ? 1 : 2;  // bytes per K/V element
   constexpr int D = 128;
@@ -462,7 +462,7 @@ __device__ __forceinline__ void mfma_attend(const AttnKP &p, const RowCtx &rc,
   long *s_q8 = L.q8;
   float &s_sq = L.sq;
 
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int lane = tid & 63, w = tid >> 6;
   const int c = lane & 15;     // V: 8-dim chunk; K: token of the round
   const int slot = lane >> 4;  // V: token slot; K: 8-dim group within 32
   const int32_t lim32 = (int32_t)min(rc.lim, (int64_t)0x7fffffff);
@@ -770,68 +770,81 @@ __global__ __launch_bounds__(SA_NT, G <= 4 ? 4 : 2) void sparse_attn_mfma_kernel
 }
 
 // The rows a tiled call (list_tile.hip) left to be attended row by row: a
-// workgroup looks at rows_per_wg rows and attends those the gate marks, part
-// by part of SA_MAX_EPS list entries (p.splits), the parts merged in
-// registers.  Usually no row is marked and the launch is the look alone.
+// workgroup looks at rows_per_wg rows, in runs of at most eight, and attends those the
+// gate marks, lists of more than SA_MAX_EPS entries part by part (p.splits).  What is
+// left are whole tiles of neighbouring queries, often the same queries of every head:
+// its runs go to different workgroups, and those of the next gridDim.x runs are turned
+// by 0.6 of that, so that these do not meet the same ones.
+// Usually no row is marked and the launch is the look alone.  The merged state of
+// the parts lies in LDS: in registers, held across mfma_attend with all that depends
+// on the lane, four heads spilled 109 of them (49 here, 42 in sparse_attn_mfma_kernel
+// itself).  Every row left, lists of 8 tokens: 4096 rows of four heads 108 us, 65
+// here (60 in sparse_attn_mfma_kernel); 16384 rows of one head 150, 108 (84).
 template <int G>
 __global__ __launch_bounds__(SA_NT, G <= 4 ? 4 : 2) void sparse_attn_gated_kernel(AttnKP p,
                                                                                   ListTileGate gt,
                                                                                   int64_t R,
                                                                                   int32_t rows_per_wg) {
+  constexpr int D = 128;
   __shared__ int32_t s_tok0[SA_MAX_EPS];
   __shared__ MfmaLds<LA_BF16, G, SA_NW> L;
-  constexpr int D = 128, NI = (G * D + SA_NT - 1) / SA_NT;
-  // lane i of every wave looks at row r0 + i (rows_per_wg <= 64)
-  const int64_t r0 = (int64_t)blockIdx.x * rows_per_wg;
+  __shared__ float s_M[G * D], s_S[G * D], s_A[G * D];  // an entry is one thread's alone
+  // lane i of every wave looks at row i of the workgroup's (rows_per_wg <= 64)
   const int lane = threadIdx.x & 63;
+  // (fewer than 2^31 rows: 2^24 tiles of 128)
+  const uint32_t turn = gridDim.x * 39u / 64u, n_rows = (uint32_t)R;
+  const int lr = rows_per_wg >= 8 ? 3 : rows_per_wg >= 4 ? 2 : rows_per_wg >= 2 ? 1 : 0;
+  const int n_look = ((rows_per_wg - 1) >> lr << lr) + (1 << lr);
+  auto row = [&](uint32_t i) {
+    const uint32_t run = i >> lr;
+    return ((run * gridDim.x + (blockIdx.x + run * turn) % gridDim.x) << lr) + (i & ((1u << lr) - 1u));
+  };
   bool mine = false;
-  if (lane < rows_per_wg && r0 + lane < R) {
-    const int64_t r = r0 + lane;
-    const int64_t t = r % p.Tq, ih = (r / p.Tq) % p.ids_heads, b = r / (p.Tq * p.ids_heads);
-    const int64_t h0 = p.ids_heads == p.Hkv ? ih * G : ih;
+  if (const uint32_t r = row(lane); lane < n_look && r < n_rows) {
+    const uint32_t bi = r / (uint32_t)p.Tq, t = r - bi * (uint32_t)p.Tq;
+    const uint32_t b = bi / (uint32_t)p.ids_heads, ih = bi - b * (uint32_t)p.ids_heads;
+    const int64_t h0 = p.ids_heads == p.Hkv ? (int64_t)ih * G : ih;
     mine = gt.dup[b * gt.m_sb + ih * gt.m_sh + t * gt.m_st] != 0 || gt.tile_left(b, h0, t);
     for (int g = 0; g < G && !mine; ++g) mine = gt.rgate[(b * p.Hq + h0 + g) * p.Tq + t] != 0;
   }
   for (uint64_t todo = __ballot(mine); todo; todo &= todo - 1) {
-    const int64_t r = r0 + __ffsll((unsigned long long)todo) - 1;
-    float M[NI], S[NI], A[NI];
-#pragma unroll
-    for (int x = 0; x < NI; ++x) {
-      M[x] = __int_as_float(0xff800000);
-      S[x] = A[x] = 0.f;
-    }
-    RowCtx rc;
+    const int64_t r = row(__ffsll((unsigned long long)todo) - 1);
     for (int64_t part = 0; part < p.splits; ++part) {
-      rc = stage_row<G, false>(p, r, part, s_tok0, nullptr);
-      mfma_attend<LA_BF16, G, false, false, SA_NW>(p, rc, s_tok0, nullptr, L);
+      // (what depends on the lane is worked out anew for each row, as in
+      // sparse_attn_mfma_kernel: held across rows it does not fit the registers)
+      int tid = threadIdx.x;
+      asm volatile("" : "+v"(tid));
+      const RowCtx rc = stage_row<G, false>(p, r, part, s_tok0, nullptr, tid);
+      mfma_attend<LA_BF16, G, false, false, SA_NW>(p, rc, s_tok0, nullptr, L, tid);
+      if (p.splits == 1) {
+        finish_row<G, D, SA_NW>(p, rc, r, 0, L.acc, L.m, L.l);
+      } else {
+        for (int i = threadIdx.x; i < G * D; i += SA_NT) {
+          const int g = i / D, d = i % D;
+          const float M = part ? s_M[i] : __int_as_float(0xff800000);
+          float mn = M;
 #pragma unroll
-      for (int x = 0; x < NI; ++x) {
-        const int i = threadIdx.x + SA_NT * x;
-        if (i >= G * D) break;
-        const int g = i / D, d = i % D;
-        float mn = M[x];
+          for (int y = 0; y < SA_NW; ++y) mn = fmaxf(mn, L.m[y][g]);
+          const float mu = mn == __int_as_float(0xff800000) ? 0.f : mn;
+          const float old = part ? fast_exp2(M - mu) : 0.f;
+          float S = part ? s_S[i] * old : 0.f, A = part ? s_A[i] * old : 0.f;
 #pragma unroll
-        for (int y = 0; y < SA_NW; ++y) mn = fmaxf(mn, L.m[y][g]);
-        const float mu = mn == __int_as_float(0xff800000) ? 0.f : mn;
-        const float old = fast_exp2(M[x] - mu);
-        S[x] *= old;
-        A[x] *= old;
-#pragma unroll
-        for (int y = 0; y < SA_NW; ++y) {
-          const float sc = fast_exp2(L.m[y][g] - mu);
-          S[x] += L.l[y][g] * sc;
-          A[x] += L.acc[y][g][d] * sc;
+          for (int y = 0; y < SA_NW; ++y) {
+            const float sc = fast_exp2(L.m[y][g] - mu);
+            S += L.l[y][g] * sc;
+            A += L.acc[y][g][d] * sc;
+          }
+          if (part + 1 < p.splits) {
+            s_M[i] = mn;
+            s_S[i] = S;
+            s_A[i] = A;
+          } else {
+            store_from_f32(p.out, rc.b * p.o_sb + (rc.h0 + g) * p.o_sh + rc.t * p.o_st + d, p.out_dt,
+                           S > 0.f ? A / S : 0.f);
+          }
         }
-        M[x] = mn;
       }
-      __syncthreads();  // the states are read before the next part's fill
-    }
-#pragma unroll
-    for (int x = 0; x < NI; ++x) {
-      const int i = threadIdx.x + SA_NT * x;
-      if (i >= G * D) break;
-      store_from_f32(p.out, rc.b * p.o_sb + (rc.h0 + i / D) * p.o_sh + rc.t * p.o_st + i % D, p.out_dt,
-                     S[x] > 0.f ? A[x] / S[x] : 0.f);
+      lds_barrier();  // the states are read before the next fill
     }
   }
 }
@@ -1237,9 +1250,9 @@ static int sparse_attention_tiles(const la_sparse_attn_args *a, const la_kv *kv,
     LA_LAUNCHED();
   }
   p.splits = ceil_div(a->N, SA_MAX_EPS);
-  // At most 64 rows a workgroup (a lane looks at each).  Where only marked rows
-  // are left 2048 workgroups do (the look alone: 5 us, 14 us with 8192); where
-  // tiles decide, whole tiles may be left and are spread over four times as many.
+  // 2048 workgroups (twice what is resident; the look alone: 5 us, 14 us with
+  // 8192), more where one would have more than 64 rows (a lane looks at each).
+  // Where many tiles may be left, four times as many, which end closer together.
   const int32_t rpw = (int32_t)std::min<int64_t>(64, ceil_div(pl.R, pl.tile.row_cost > 0.f ? 8192 : 2048));
   const dim3 grid((unsigned)ceil_div(pl.R, rpw));
   switch (pl.G) {

@@ -131,6 +131,23 @@ def test_tiles_leave_units_listed_twice_to_the_rows(dev, unit):
     _check(got, want, 2e-6)
 
 
+@pytest.mark.parametrize("G", [1, 2, 4, 8])
+def test_long_lists_left_to_the_rows_in_parts(dev, G):
+    """More than 1024 entries: the row kernel takes a left row's list in parts; some
+    rows' counts leave a part, or all of them, empty."""
+    Tq = 130 * 8 // G + 3
+    q, k, v = _inputs(1, 2, G, Tq, 2000)
+    ids = _lists(1, 2, Tq, 2000, 1, 0.9)
+    ids[:, :, ::2, 0] = ids[:, :, ::2, 1]
+    g = torch.Generator().manual_seed(4)
+    counts = torch.randint(2, ids.shape[-1] + 1, ids.shape[:3], generator=g).to(torch.int32)
+    counts[:, :, 4:8] = torch.tensor([0, 1, 900, 1025], dtype=torch.int32)
+    ids[:, :, :2] = -1
+    got = _run(dev, q, k, v, ids, unit=1, counts=counts, out_dtype=torch.float32)
+    want = oracle.attend_lists(q, k, v, ids.numpy(), unit=1, counts=counts.numpy())
+    _check(got, want, 2e-6)
+
+
 def test_tiles_keep_unlisted_values_out(dev):
     """Infinities, NaN and huge values reach only the rows that list them."""
     q, k, v = _inputs(1, 2, 4, 300, 1000)

@@ -45,6 +45,14 @@ typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
 constexpr int LT_M = 128, LT_NT = 256, LT_NW = 4, LT_D = 128, LT_BS = 64;
 constexpr int LT_BLK = LT_BS * LT_D;   // elements of a staged K or V block
 constexpr int LT_MAXB = 4096;          // key blocks of a cache (list positions in LDS)
+// Tiles are left where that is clearly cheaper: both costs are good to a fifth, and
+// left rows start when the tiles have ended.  Up to LT_ONE tiles are left together:
+// they run at the same time, and as long as any of them when others are left (1024
+// queries of 16 heads, 128 tokens of 8192 a row: 147 us in tiles, 137 in rows, 197 with
+// half of the tiles left).
+constexpr float LT_LEAVE = 1.25f;
+constexpr int64_t LT_ONE = 4096;
+enum { LT_TILES, LT_EACH, LT_TOGETHER };  // who decides: nobody, each tile, all of them
 
 // Chunk swizzles of staged row r (16-byte chunks, 16 per row).  K: the 8-lane
 // groups a ds_read_b128 pass serves together ({0,3}, {1,2}, ...) hold rows 8i..8i+7
@@ -60,6 +68,7 @@ struct LmKP {
   int64_t id_sb, id_sh, id_st, N, unit, T;
   int64_t ids_heads, ids_rows, mheads, mrows;
   int32_t nblk, token, rw, lw;  // rw: mask rows per workgroup, lw: LDS words per row
+  unsigned long long *balance;  // (set to 0 for list_union_kernel)
 };
 
 __global__ __launch_bounds__(256) void list_mask_kernel(LmKP p) {
@@ -69,6 +78,7 @@ __global__ __launch_bounds__(256) void list_mask_kernel(LmKP p) {
   const int64_t row0 = (int64_t)blockIdx.x * p.rw;
   for (int i = tid; i < p.rw * p.lw; i += 256) lbits[i] = 0u;
   if (tid < 32) s_dup[tid] = 0u;
+  if (blockIdx.x == 0 && tid == 0) *p.balance = 0ull;
   __syncthreads();
   const int tpr = 256 / p.rw;  // threads of a row
   const int rl = tid / tpr, tl = tid % tpr;
@@ -134,15 +144,18 @@ struct LtKP {
   const uint32_t *mask;
   uint16_t *list;   // [tile][nblk]: the blocks its rows list, ascending
   int32_t *nlist;   // [tile]: how many; -1: the tile is left to the row kernel
+  // LT_TOGETHER: what walking costs more than the rows, summed over the tiles (two's
+  // complement), which decides for all of them; else null
+  unsigned long long *balance;
   uint8_t *rgate;   // [b][h][t]: a row whose result is not finite
-  const int32_t *kv_len;
+  const int32_t *kv_len, *counts;
   float *ws_ml, *ws_acc;
   int64_t q_sb, q_sh, q_st, o_sb, o_sh, o_st;
   int64_t k_sb, k_sh, k_st, v_sb, v_sh, v_st;
   int64_t mrows, m_sb, m_sh, m_st, T, offset;
   int32_t Hq, Hkv, Tq, G, gt, qt, ntile, ngrp, nblk, splits, per_head, causal, out_dt, vec_out;
-  int32_t ids_heads, nstream;
-  float qscale, thr_gap, row_cost;  // row_cost > 0: tiles decide (see list_union_kernel)
+  int32_t ids_heads, nstream, N, unit, decide;
+  float qscale, thr_gap, row_fixed, row_tok;  // row_*: see list_union_kernel
 };
 
 // Last key any query of the tile [t0, tl] may read, and its blocks.
@@ -152,14 +165,13 @@ __device__ __forceinline__ int lt_blocks(const LtKP &p, int64_t len, int tl) {
 }
 
 // One workgroup per tile: the blocks any of its rows lists, within reach.
-// With row_cost > 0 the tile is left to the row kernel (count -1) when walking
-// them for all 128 rows costs more than the listed tokens row by row, in units
-// of a row and token of a walked block (a shared list is read once for its
-// heads there).
+// The tile is left to the row kernel (count -1) when walking them for all 128 rows
+// costs more than the lists row by row, entry by entry as that kernel walks them
+// (to their counts, -1 entries too), by LT_LEAVE, in units of a row and token of a
+// walked block (a shared list is read once for its heads there).
 template <bool TOKEN>
 __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
   __shared__ uint32_t s_union[LT_MAXB / 32];
-  __shared__ uint32_t s_cnt[LT_NW];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int64_t tg = blockIdx.x;  // (b, group, tile)
   const int tile = (int)(tg % p.ntile), grp = (int)((tg / p.ntile) % p.ngrp);
@@ -179,7 +191,12 @@ __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
     mr[x] = p.m_st == 0 ? mbase + i * p.m_sh : mbase + (int64_t)(i / nq) * p.m_sh + t0 + i % nq;
   }
   const bool in0 = lane < nr, in1 = lane + 64 < nr;
-  uint32_t listed = 0;
+  // their list entries (with counts, mask rows are numbered as those are)
+  int32_t ne[2] = {in0 ? p.N : 0, in1 ? p.N : 0};
+  if (p.decide != LT_TILES && p.counts && w == 0) {
+    if (in0) ne[0] = min(ne[0], max(p.counts[mr[0]], 0));
+    if (in1) ne[1] = min(ne[1], max(p.counts[mr[1]], 0));
+  }
   for (int x = w; x * 32 < nb; x += LT_NW) {
     uint32_t word = 0;
     if constexpr (TOKEN) {
@@ -196,7 +213,6 @@ __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           if (k0 + e >= kbe) break;
-          listed += __popc(v[e].x) + __popc(v[e].y) + __popc(u[e].x) + __popc(u[e].y);
           if (__ballot((v[e].x | v[e].y | u[e].x | u[e].y) != 0) != 0) word |= 1u << (k0 + e);
         }
       }
@@ -204,16 +220,12 @@ __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
       const uint32_t in_nb = nb - 32 * x >= 32 ? 0xffffffffu : (1u << (nb - 32 * x)) - 1u;
       const uint32_t y = in0 ? p.mask[(int64_t)x * p.mrows + mr[0]] & in_nb : 0u;
       const uint32_t z = in1 ? p.mask[(int64_t)x * p.mrows + mr[1]] & in_nb : 0u;
-      listed += LT_BS * (__popc(y) + __popc(z));
       word = y | z;
 #pragma unroll
       for (int o = 32; o >= 1; o >>= 1) word |= (uint32_t)__shfl_xor((int)word, o, 64);
     }
     if (lane == 0) s_union[x] = word;
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) listed += (uint32_t)__shfl_xor((int)listed, o, 64);
-  if (lane == 0) s_cnt[w] = listed;
   __syncthreads();
   if (w != 0) return;
   constexpr int WPL = LT_MAXB / 32 / 64;
@@ -231,9 +243,17 @@ __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
     if (lane >= o) incl += y;
   }
   const uint32_t total = (uint32_t)__shfl((int)incl, 63, 64);
-  const float row_work = p.row_cost * (float)(s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3]) *
-                         (p.m_st == 0 ? (float)nq : 1.f);
-  const bool rows = p.row_cost > 0.f && (float)total * (float)(LT_M * LT_BS) > row_work;
+  bool rows = false;
+  if (p.decide != LT_TILES) {
+    float entries = (float)ne[0] + (float)ne[1];
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) entries += __shfl_xor(entries, o, 64);
+    const float row_work = (p.row_fixed * (float)nr + p.row_tok * entries * (float)p.unit) *
+                           (p.m_st == 0 ? (float)nq : 1.f);
+    const float over = (float)total * (float)(LT_M * LT_BS) - LT_LEAVE * row_work;
+    rows = p.decide == LT_EACH && over > 0.f;
+    if (p.decide == LT_TOGETHER && lane == 0) atomicAdd(p.balance, (unsigned long long)(long long)over);
+  }
   if (lane == 0) p.nlist[tg] = rows ? -1 : (int32_t)total;
   if (rows) return;
   uint16_t *out = p.list + tg * p.nblk;
@@ -279,7 +299,7 @@ __global__ __launch_bounds__(LT_NT, 2) void list_tile_kernel(LtKP p) {
   const int64_t mbase = b * p.m_sb + (int64_t)(p.per_head ? h0 : h0 / p.G) * p.m_sh;
   const int64_t tg = (b * p.ngrp + grp) * p.ntile + tile;
   const int nall = p.nlist[tg];
-  if (nall < 0) return;  // left to the row kernel
+  if (nall < 0 || (p.balance && (long long)*p.balance > 0)) return;  // left to the row kernel
   const int e0 = (int)((int64_t)nall * split / p.splits);
   const int n = (int)((int64_t)nall * (split + 1) / p.splits) - e0;
   for (int i = tid; i < n; i += LT_NT) s_list[i] = p.list[tg * p.nblk + e0 + i];
@@ -527,16 +547,31 @@ __global__ __launch_bounds__(LT_NT, 2) void list_tile_kernel(LtKP p) {
 
 static size_t up256(size_t x) { return (x + 255) / 256 * 256; }
 
-// Cost of a listed token of one list row in the row kernels, in picoseconds of
-// the whole device, by the heads that share the list (512 queries, 8 KV heads,
-// 16384 keys: 47 / 51 / 120 / 76 measured), against LT_TILE_PS for a row and
-// token of a walked block here (0.93-1.06 measured with every CU busy).
-static float row_ps(int64_t heads) { return heads == 4 ? 110.f : heads == 8 ? 70.f : 45.f; }
-constexpr float LT_TILE_PS = 1.1f;
+// Cost of a list row in the row kernels, in picoseconds of the whole device: of the
+// row, and of each token of its list, by the heads that share it.  Fits of 64 to 2048
+// tokens a row to a tenth (512 queries of 8 KV heads and 4096 keys, 2048 queries of 2
+// or 8 and 16384 keys, units of 1, 8 and 64); over 65536 keys, which miss the L2s, 1.2
+// (4 heads) to 1.7 (1 head) times as much a token.  (Four heads cost more a token than
+// eight: held to four waves a SIMD their kernel spills 42 registers.)  Against
+// LT_TILE_PS for a row and token of a walked block here (0.93-1.06 measured with
+// every CU busy).  A row that its tile leaves costs LT_LEFT_PS more: its workgroup
+// takes several one after another (16384 rows of one head and 32 tokens: 84 us in
+// sparse_attn_mfma_kernel, 108 in sparse_attn_gated_kernel).
+struct RowCost {
+  float fixed, tok;
+};
+static RowCost row_ps(int64_t heads) {
+  return heads == 8 ? RowCost{14000.f, 59.f} : heads == 4 ? RowCost{10000.f, 103.f}
+         : heads == 2 ? RowCost{7000.f, 41.f} : RowCost{4000.f, 38.f};
+}
+constexpr float LT_TILE_PS = 1.1f, LT_LEFT_PS = 2000.f;
 // The masks, the merge and the look for marked rows cost about 25 us here, so
 // calls the row kernels finish sooner stay with them (measured, 512 listed
 // tokens per query, 8 heads: 128 queries 34 us by rows, 43 by tiles; 512
-// queries 93 and 50).
+// queries 93 and 50).  The host knows the width of lists, not their counts: wide lists
+// that turn out nearly empty pay those 25 us and the dearer rows (512 queries of 8
+// lists over 8192 keys, units of 8: 1 unit a list 60 us by rows, 72 here, 4 units 62 and
+// 94, 16 units 100 and 130; 64 units 247 and 154, full lists 1400 and 116).
 constexpr float LT_MIN_ROW_US = 40.f;
 
 ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
@@ -560,8 +595,9 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
     const double n = (double)a->Tq, x = std::min(std::max(cap - o, 0.0), n);
     return (x * (o + (x + 1) / 2) + (n - x) * cap) / n;
   };
-  const double rows_ps = (double)(a->B * a->ids_heads * a->Tq) * row_ps(per_head ? 1 : G) *
-                         mean((double)std::min(a->N * a->unit, kv->T));
+  const RowCost rc = row_ps(per_head ? 1 : G);
+  const double rows_ps = (double)(a->B * a->ids_heads * a->Tq) *
+                         (rc.fixed + rc.tok * mean((double)std::min(a->N * a->unit, kv->T)));
   const int64_t gt = pow2 ? G : 1, qt = LT_M / gt;
   const double tile_ps = (double)(a->B * (a->Hq / gt) * ceil_div(a->Tq, qt) * LT_M) * LT_TILE_PS * mean((double)kv->T);
   if (rows_ps < LT_MIN_ROW_US * 1e6) return pl;
@@ -571,7 +607,9 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
   // drawing from the same 68 blocks: 269 us by rows, 109 by tiles).
   const bool sure = tile_ps < 0.9 * rows_ps;
   if (!sure && (a->unit % LT_BS != 0 || reach > 64 * a->N * a->unit)) return pl;
-  pl.row_cost = sure ? 0.f : row_ps(per_head ? 1 : G) / LT_TILE_PS;
+  pl.sure = sure;
+  pl.row_fixed = (rc.fixed + LT_LEFT_PS) / LT_TILE_PS;
+  pl.row_tok = rc.tok / LT_TILE_PS;
   pl.gt = (int32_t)gt;
   pl.qt = (int32_t)qt;
   pl.ntile = (int32_t)ceil_div(a->Tq, pl.qt);
@@ -586,6 +624,12 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
   pl.m_sh = one_h ? 0 : a->ids_rows;
   pl.m_sb = one_b ? 0 : mh * a->ids_rows;
   const int64_t tiles = a->B * pl.ngrp * pl.ntile;
+  // Nothing to decide where even walking every block beats rows whose counts are 0 (or
+  // whose lists, without counts, are walked to the end).
+  const double least_ps = (double)(a->B * a->ids_heads * a->Tq) *
+                          (rc.fixed + LT_LEFT_PS + (a->counts ? 0.0 : rc.tok * (double)(a->N * a->unit)));
+  pl.decide = !sure ? LT_EACH : tile_ps < LT_LEAVE * least_ps ? LT_TILES
+              : tiles <= LT_ONE ? LT_TOGETHER : LT_EACH;
   if (tiles > ((int64_t)1 << 24) || pl.mrows > ((int64_t)1 << 30)) return pl;
   // two workgroups per CU; parts of at least 8 blocks
   const int64_t want = ceil_div((int64_t)2 * num_cus(), tiles);
@@ -600,6 +644,7 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
   pl.off_dup = take((size_t)pl.mrows);
   pl.off_list = take((size_t)tiles * pl.nblk * 2);
   pl.off_nlist = take((size_t)tiles * 4);
+  pl.off_balance = take(sizeof(uint64_t));
   pl.off_rgate = take((size_t)(a->B * a->Hq * a->Tq));
   if (pl.splits > 1) {
     const size_t parts = (size_t)(a->B * a->Hq * a->Tq) * pl.splits;
@@ -627,6 +672,7 @@ int list_tile_launch(const la_sparse_attn_args *a, const la_kv *kv, const ListTi
   m.mrows = pl.mrows;
   m.nblk = pl.nblk;
   m.token = pl.token;
+  m.balance = (unsigned long long *)(base + pl.off_balance);
   m.lw = (int32_t)(pl.token ? 2 * pl.nblk : ceil_div(pl.nblk, 32));
   m.rw = 32;
   // rows share a workgroup (and write their masks side by side) as long as
@@ -645,8 +691,11 @@ int list_tile_launch(const la_sparse_attn_args *a, const la_kv *kv, const ListTi
   p.mask = m.mask;
   p.list = (uint16_t *)(base + pl.off_list);
   p.nlist = (int32_t *)(base + pl.off_nlist);
+  p.decide = pl.decide;
+  p.balance = pl.decide == LT_TOGETHER ? m.balance : nullptr;
   p.rgate = base + pl.off_rgate;
   p.kv_len = kv->kv_len;
+  p.counts = a->counts;
   if (pl.splits > 1) {
     p.ws_ml = (float *)(base + pl.off_ml);
     p.ws_acc = (float *)(base + pl.off_acc);
@@ -668,10 +717,13 @@ int list_tile_launch(const la_sparse_attn_args *a, const la_kv *kv, const ListTi
   const int64_t oal = a->out_dtype == LA_F32 ? 16 : 8;
   p.vec_out = (uintptr_t)a->out % oal == 0 && a->o_sb % 4 == 0 && a->o_sh % 4 == 0 && a->o_st % 4 == 0;
   p.ids_heads = (int32_t)a->ids_heads;
+  p.N = (int32_t)a->N;
+  p.unit = (int32_t)a->unit;
   p.nstream = (int32_t)(a->B * pl.ngrp * pl.splits);
   p.qscale = a->scale * 1.4426950408889634f;
   p.thr_gap = 8.f / p.qscale;
-  p.row_cost = pl.row_cost;
+  p.row_fixed = pl.row_fixed;
+  p.row_tok = pl.row_tok;
   const int64_t tiles = a->B * pl.ngrp * pl.ntile;
   const dim3 grid((unsigned)(tiles * pl.splits));
   if (pl.token) {
@@ -684,7 +736,7 @@ int list_tile_launch(const la_sparse_attn_args *a, const la_kv *kv, const ListTi
     list_tile_kernel<false><<<grid, LT_NT, 0, st>>>(p);
   }
   LA_LAUNCHED();
-  gate = ListTileGate{m.dup, p.rgate, p.nlist, pl.m_sb, pl.m_sh, pl.m_st,
+  gate = ListTileGate{m.dup, p.rgate, p.nlist, p.balance, pl.m_sb, pl.m_sh, pl.m_st,
                       pl.qt, pl.ntile, pl.ngrp, pl.gt};
   return LA_OK;
 }

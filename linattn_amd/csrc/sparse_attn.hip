@@ -1253,7 +1253,7 @@ static int sparse_attention_tiles(const la_sparse_attn_args *a, const la_kv *kv,
   // 2048 workgroups (twice what is resident; the look alone: 5 us, 14 us with
   // 8192), more where one would have more than 64 rows (a lane looks at each).
   // Where many tiles may be left, four times as many, which end closer together.
-  const int32_t rpw = (int32_t)std::min<int64_t>(64, ceil_div(pl.R, pl.tile.row_cost > 0.f ? 8192 : 2048));
+  const int32_t rpw = (int32_t)std::min<int64_t>(64, ceil_div(pl.R, pl.tile.sure ? 2048 : 8192));
   const dim3 grid((unsigned)ceil_div(pl.R, rpw));
   switch (pl.G) {
     case 1: sparse_attn_gated_kernel<1><<<grid, SA_NT, 0, st>>>(p, gate, pl.R, rpw); break;

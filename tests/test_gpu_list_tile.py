@@ -176,6 +176,25 @@ def test_tiles_that_share_little_go_to_the_rows(dev):
     _check(got, want, 2e-6)
 
 
+@pytest.mark.parametrize("unit,per_head,given", [(8, False, "counts"), (8, True, "pad"),
+                                                 (64, True, "counts"), (1, False, "counts")])
+def test_wide_lists_decide_by_what_they_hold(dev, unit, per_head, given):
+    """Lists as wide as the cache, of which tiles of rows use a few entries or all."""
+    q, k, v = _inputs(1, 2, 4, 400, 3000)
+    ids = _lists(1, 8 if per_head else 2, 400, 3000, unit, 1.0)
+    counts = torch.full(ids.shape[:3], ids.shape[-1], dtype=torch.int32)
+    counts[:, :, :130] = 3
+    counts[:, :, 130:256] = 0
+    counts[:, :, 300:310] = 1
+    if given == "pad":
+        ids = torch.where(torch.arange(ids.shape[-1]) < counts[..., None], ids, -1)
+        counts = None
+    got = _run(dev, q, k, v, ids, unit=unit, counts=counts, out_dtype=torch.float32)
+    want = oracle.attend_lists(q, k, v, ids.numpy(), unit=unit,
+                               counts=None if counts is None else counts.numpy())
+    _check(got, want, 2e-6)
+
+
 def test_small_calls_and_given_splits_stay_with_the_rows(dev):
     q, k, v = _inputs(1, 2, 4, 300, 1000)
     ids = _lists(1, 8, 300, 1000, 1, 0.6)

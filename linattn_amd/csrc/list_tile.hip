@@ -142,6 +142,7 @@ struct LtKP {
   const uint16_t *q, *k, *v;
   void *out;
   const uint32_t *mask;
+  const uint8_t *dup;
   uint16_t *list;   // [tile][nblk]: the blocks its rows list, ascending
   int32_t *nlist;   // [tile]: how many; -1: the tile is left to the row kernel
   // LT_TOGETHER: what walking costs more than the rows, summed over the tiles (two's
@@ -168,7 +169,8 @@ __device__ __forceinline__ int lt_blocks(const LtKP &p, int64_t len, int tl) {
 // The tile is left to the row kernel (count -1) when walking them for all 128 rows
 // costs more than the lists row by row, entry by entry as that kernel walks them
 // (to their counts, -1 entries too), by LT_LEAVE, in units of a row and token of a
-// walked block (a shared list is read once for its heads there).
+// walked block (a shared list is read once for its heads there); or when every row
+// lists a unit twice.
 template <bool TOKEN>
 __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
   __shared__ uint32_t s_union[LT_MAXB / 32];
@@ -193,9 +195,13 @@ __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
   const bool in0 = lane < nr, in1 = lane + 64 < nr;
   // their list entries (with counts, mask rows are numbered as those are)
   int32_t ne[2] = {in0 ? p.N : 0, in1 ? p.N : 0};
-  if (p.decide != LT_TILES && p.counts && w == 0) {
-    if (in0) ne[0] = min(ne[0], max(p.counts[mr[0]], 0));
-    if (in1) ne[1] = min(ne[1], max(p.counts[mr[1]], 0));
+  bool once = false;  // one of them lists no unit twice
+  if (w == 0) {
+    once = (in0 && p.dup[mr[0]] == 0) || (in1 && p.dup[mr[1]] == 0);
+    if (p.decide != LT_TILES && p.counts) {
+      if (in0) ne[0] = min(ne[0], max(p.counts[mr[0]], 0));
+      if (in1) ne[1] = min(ne[1], max(p.counts[mr[1]], 0));
+    }
   }
   for (int x = w; x * 32 < nb; x += LT_NW) {
     uint32_t word = 0;
@@ -243,8 +249,8 @@ __global__ __launch_bounds__(LT_NT) void list_union_kernel(LtKP p) {
     if (lane >= o) incl += y;
   }
   const uint32_t total = (uint32_t)__shfl((int)incl, 63, 64);
-  bool rows = false;
-  if (p.decide != LT_TILES) {
+  bool rows = __ballot(once) == 0;  // (every row would be done again)
+  if (p.decide != LT_TILES && !rows) {
     float entries = (float)ne[0] + (float)ne[1];
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) entries += __shfl_xor(entries, o, 64);
@@ -689,6 +695,7 @@ int list_tile_launch(const la_sparse_attn_args *a, const la_kv *kv, const ListTi
   p.v = (const uint16_t *)kv->v;
   p.out = a->out;
   p.mask = m.mask;
+  p.dup = m.dup;
   p.list = (uint16_t *)(base + pl.off_list);
   p.nlist = (int32_t *)(base + pl.off_nlist);
   p.decide = pl.decide;

@@ -131,6 +131,22 @@ def test_tiles_leave_units_listed_twice_to_the_rows(dev, unit):
     _check(got, want, 2e-6)
 
 
+@pytest.mark.parametrize("unit,per_head", [(1, True), (1, False), (64, True)])
+def test_tiles_whose_every_row_lists_a_unit_twice(dev, unit, per_head):
+    """Whole tiles (32 queries), all but one row of one, and one list for every query."""
+    q, k, v = _inputs(1, 2, 4, 400, 1000)
+    ids = _lists(1, 8 if per_head else 2, 400, 1000, unit, 0.6)
+    ids[..., 1] = ids[..., 0] = 3
+    ids[:, 1, 40, 1] = -1
+    ids[:, :, 64:130, 1] = -1
+    got = _run(dev, q, k, v, ids, unit=unit, out_dtype=torch.float32)
+    want = oracle.attend_lists(q, k, v, ids.numpy(), unit=unit)
+    _check(got, want, 2e-6)
+    one = ids[:, :, :1].contiguous()
+    got = _run(dev, q, k, v, one, unit=unit, out_dtype=torch.float32)
+    _check(got, oracle.attend_lists(q, k, v, one.numpy(), unit=unit), 2e-6)
+
+
 @pytest.mark.parametrize("G", [1, 2, 4, 8])
 def test_long_lists_left_to_the_rows_in_parts(dev, G):
     """More than 1024 entries: the row kernel takes a left row's list in parts; some

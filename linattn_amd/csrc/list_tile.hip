@@ -30,6 +30,7 @@
 // each is the exact sum of three bf16 terms (8 significant bits each), one
 // product per term, so the result is the fp32 one (V and q, k are bf16 already).
 #include <algorithm>
+#include <numeric>
 
 #include "kv_access.h"
 #include "list_tile.h"
@@ -580,12 +581,36 @@ constexpr float LT_TILE_PS = 1.1f, LT_LEFT_PS = 2000.f;
 // 94, 16 units 100 and 130; 64 units 247 and 154, full lists 1400 and 116).
 constexpr float LT_MIN_ROW_US = 40.f;
 
+// Whether out may share memory with q: rows done again read q after their tile has
+// stored (a row kernel reads a row of q before it writes that row of out).  Not where
+// the spans of the two are apart, nor where rows lie in different places of what all
+// strides are multiples of (halves of one tensor).
+static bool out_in_q(const la_sparse_attn_args *a) {
+  const int64_t eo = a->out_dtype == LA_F32 ? 4 : 2, nq = a->D * 2, no = a->D * eo;  // (q is bf16)
+  const int64_t step[3][2] = {{a->q_sb * 2, a->o_sb * eo}, {a->q_sh * 2, a->o_sh * eo}, {a->q_st * 2, a->o_st * eo}};
+  const int64_t count[3] = {a->B, a->Hq, a->Tq};
+  int64_t g = 0, q0 = (int64_t)(uintptr_t)a->q, o0 = (int64_t)(uintptr_t)a->out;
+  const int64_t d = o0 - q0;
+  int64_t q1 = q0 + nq, o1 = o0 + no;
+  for (int x = 0; x < 3; ++x) {
+    if (count[x] == 1) continue;
+    for (const int64_t s : {step[x][0], step[x][1]}) g = std::gcd(g, s);
+    (step[x][0] < 0 ? q0 : q1) += (count[x] - 1) * step[x][0];
+    (step[x][1] < 0 ? o0 : o1) += (count[x] - 1) * step[x][1];
+  }
+  if (o0 >= q1 || q0 >= o1) return false;
+  if (g == 0) return true;
+  const int64_t at = ((d % g) + g) % g;  // a row of out, past a row of q
+  return !(at >= nq && g - at >= no);
+}
+
 ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
   ListTilePlan pl;
   if (kv->page_table || kv->dtype != LA_BF16 || a->q_dtype != LA_BF16 || a->D != LT_D ||
       a->num_splits > 0 || !(a->scale > 0.f) || a->scale > 64.f)
     return pl;
   auto m8 = [](int64_t x) { return x % 8 == 0; };
+  if (out_in_q(a)) return pl;
   if ((uintptr_t)a->q % 16 || !m8(a->q_sb) || !m8(a->q_sh) || !m8(a->q_st)) return pl;
   if (a->Tq < 32 || kv->T > (int64_t)LT_MAXB * LT_BS || a->offset < 0) return pl;
   const int64_t lim_st = (int64_t)1 << 23;  // 32-bit byte offsets of a block's rows

@@ -220,3 +220,24 @@ def test_small_calls_and_given_splits_stay_with_the_rows(dev):
     few = _run(dev, q[:, :, :31], k, v, ids[:, :, :31].contiguous(), unit=1, tiled=None,
                out_dtype=torch.float32)
     _check(few, rows[:, :, :31], 2e-6)
+
+
+def test_out_may_be_q(dev):
+    """Written over q (or over what q starts in), each row is read before it is written,
+    rows done again too."""
+    q, k, v = _inputs(1, 2, 4, 300, 1000)
+    ids = _lists(1, 8, 300, 1000, 1, 0.6)
+    ids[:, :, 5::7, 0] = ids[:, :, 5::7, 1]
+    kw = dict(unit=1, out_dtype=torch.bfloat16)
+    want = _run(dev, q, k, v, ids, **kw)
+    qd = q.to(dev)
+    got = _run(dev, qd, k, v, ids, unit=1, out=qd, tiled=False)
+    _check(got, want, 3e-3)
+    both = torch.zeros(1, 8, 300, 256, dtype=torch.bfloat16, device=dev)
+    both[..., :128] = q.to(dev)  # side by side: nothing shared
+    got = _run(dev, both[..., :128], k, v, ids, unit=1, out=both[..., 128:])
+    _check(got, want, 3e-3)
+    assert torch.equal(both[..., :128].cpu(), q)
+    late = torch.zeros(1, 8, 301, 128, dtype=torch.bfloat16, device=dev)
+    late[:, :, 1:] = q.to(dev)  # a query further on: rows of q are other rows of out
+    _run(dev, late[:, :, 1:], k, v, ids, unit=1, out=late[:, :, :-1], tiled=False)

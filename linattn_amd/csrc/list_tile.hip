@@ -580,6 +580,8 @@ constexpr float LT_TILE_PS = 1.1f, LT_LEFT_PS = 2000.f;
 // lists over 8192 keys, units of 8: 1 unit a list 60 us by rows, 72 here, 4 units 62 and
 // 94, 16 units 100 and 130; 64 units 247 and 154, full lists 1400 and 116).
 constexpr float LT_MIN_ROW_US = 40.f;
+// Masks, block lists, marks and parts of one call (the row kernels need none of it).
+constexpr size_t LT_MAX_BYTES = (size_t)512 << 20;
 
 // Whether out may share memory with q: rows done again read q after their tile has
 // stored (a row kernel reads a row of q before it writes that row of out).  Not where
@@ -668,7 +670,6 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
   const size_t words = pl.token ? (size_t)pl.nblk * 2 : (size_t)ceil_div(pl.nblk, 32);
   if (pl.token && words * 4 > 49152) return pl;
   const size_t mask = words * 4 * (size_t)pl.mrows;
-  if (mask > ((size_t)1 << 29)) return pl;
   size_t at = 0;
   auto take = [&](size_t n) { const size_t o = at; at += up256(n); return o; };
   pl.off_mask = take(mask);
@@ -682,6 +683,7 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
     pl.off_ml = take(parts * 2 * sizeof(float));
     pl.off_acc = take(parts * LT_D * sizeof(float));
   }
+  if (at > LT_MAX_BYTES) return pl;
   pl.bytes = at;
   pl.use = true;
   return pl;

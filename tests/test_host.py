@@ -115,3 +115,28 @@ def test_head_selection_refuses_what_its_grid_cannot_hold():
 def test_head_selection_takes_the_faster_form(rows, pages, k, D, G, one):
     from linattn_amd.kernels.quest_pages import _heads_in_one_kernel
     assert _heads_in_one_kernel(rows, pages, k, D, G) is one
+
+
+@pytest.mark.parametrize("tq,tiled", [(8192, True), (32768, False)])
+def test_list_tiles_bound_their_workspace(tq, tiled):
+    """Tiles of many queries over a long cache, whose block lists grow with both: within
+    512 MiB, or the row kernels (which need no workspace for so many rows)."""
+    import ctypes
+
+    from linattn_amd import _native as N
+    a, kv = N.LaSparseAttnArgs(), N.LaKV()
+    B, H, T, D = 64, 8, 262144, 128
+    a.q, a.out, a.ids = 1 << 40, 1 << 44, 1 << 46  # (never read)
+    a.B, a.Hq, a.Hkv, a.Tq, a.D = B, H, H, tq, D
+    a.q_sb = a.o_sb = H * tq * D
+    a.q_sh = a.o_sh = tq * D
+    a.q_st = a.o_st = D
+    a.ids_heads, a.ids_rows, a.N, a.unit = H, tq, 512, 64
+    a.id_sb = a.id_sh = 0
+    a.id_st, a.scale, a.q_dtype, a.out_dtype = 512, 0.1, N.LA_BF16, N.LA_BF16
+    kv.k, kv.v, kv.T, kv.dtype = 1 << 47, 1 << 48, T, N.LA_BF16
+    kv.k_sb = kv.v_sb = H * T * D
+    kv.k_sh = kv.v_sh = T * D
+    kv.k_st = kv.v_st = D
+    n = N.load().la_sparse_attention_workspace(ctypes.byref(a), ctypes.byref(kv))
+    assert (256 << 20) < n <= (512 << 20) if tiled else n == 0

@@ -70,10 +70,12 @@ def _check(got, want, tol):
     assert np.isfinite(got).all()
     err = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert err < tol, err
-    # no row is off by itself: each within 4 times its share
-    rows = np.linalg.norm(got - want, axis=-1)
-    scale = np.linalg.norm(want) / np.sqrt(rows.size)
-    assert rows.max() < 8 * tol * scale, rows.max() / scale
+    # no row is off by itself: each within the bar of its own norm (rows of few keys are
+    # long, and rounding is relative) and 4 times that of the average row (rows of many
+    # keys are short: their terms cancel, their errors do not)
+    rows, own = np.linalg.norm(got - want, axis=-1), np.linalg.norm(want, axis=-1)
+    bar = tol * (own + 4 * np.linalg.norm(want) / np.sqrt(rows.size))
+    assert (rows < bar).all(), (rows / bar).max()
 
 
 @pytest.mark.parametrize("G,per_head,Tq,T,unit", [
@@ -241,3 +243,28 @@ def test_out_may_be_q(dev):
     late = torch.zeros(1, 8, 301, 128, dtype=torch.bfloat16, device=dev)
     late[:, :, 1:] = q.to(dev)  # a query further on: rows of q are other rows of out
     _run(dev, late[:, :, 1:], k, v, ids, unit=1, out=late[:, :, :-1], tiled=False)
+
+
+def test_tiles_replay_in_a_graph(dev):
+    """Captured once, replayed over other inputs between eager calls: lists that run as
+    tiles, lists that tiles leave (short, or with a unit twice), and back."""
+    q, k, v = _inputs(1, 2, 4, 400, 3000)
+    full = _lists(1, 2, 400, 3000, 8, 1.0)
+    twice = full.clone()
+    twice[:, :, ::3, 5] = twice[:, :, ::3, 6]
+    many = torch.full(full.shape[:3], full.shape[-1], dtype=torch.int32)
+    cases = [(full, many), (full, torch.full_like(many, 2)), (twice, many // 2), (full, many // 3)]
+    want = [oracle.attend_lists(q, k, v, i.numpy(), unit=8, counts=c.numpy()) for i, c in cases]
+    qd, kd, vd, ids, counts = (x.to(dev).clone() for x in (q, k, v, *cases[0]))
+    _run(dev, qd, kd, vd, ids, unit=8, counts=counts, out_dtype=torch.float32)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = sparse_attention(qd, kd, vd, ids, unit=8, counts=counts, out_dtype=torch.float32)
+    for i in (0, 1, 2, 3, 1, 0):
+        ids.copy_(cases[i][0])
+        counts.copy_(cases[i][1])
+        out.zero_()
+        graph.replay()
+        eager = sparse_attention(qd, kd, vd, ids, unit=8, counts=counts, out_dtype=torch.float32)
+        _check(out.cpu().double().numpy(), want[i], 2e-6)
+        assert torch.equal(out, eager)

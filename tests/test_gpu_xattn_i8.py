@@ -16,14 +16,11 @@ SHAPES = [  # B, Hq, Hkv, Tq, T, D, block, offset: from 256 key blocks and 512 t
     (2, 18, 2, 1030, 1030, 128, 4, 0),     # a partial last block and tile
     (1, 36, 4, 530, 530, 64, 2, 0),
     (2, 32, 8, 650, 2600, 64, 8, 1950),    # queries at an offset
-    (1, 24, 8, 1030, 4110, 128, 16, 3080),
+    (2, 28, 4, 1030, 4110, 128, 16, 3080),  # the largest block
 ]
 
 
-@pytest.mark.parametrize("data", ["normal", "few", "wide", "special"])
-@pytest.mark.parametrize("shape", SHAPES)
-def test_int8_slots_select_as_fp64(shape, data):
-    from linattn_amd.kernels.routing import xattn_select_hip
+def _inputs(shape, data):
     B, Hq, Hkv, Tq, T, D, blk, off = shape
     g = torch.Generator().manual_seed(T + D)
     q = torch.randn(B, Tq, Hq, D, generator=g)
@@ -40,15 +37,72 @@ def test_int8_slots_select_as_fp64(shape, data):
         k[:, :, 40, 5] = float("nan")
         k[:, :, 41, 6] = -float("inf")
         k[:, :, 50] = 1e-40  # denormal
-    q = q.bfloat16().cuda().transpose(1, 2)  # [B, Hq, Tq, D] over [B, Tq, Hq, D]
-    k = k.bfloat16().cuda()
-    n_kb = -(-T // blk)
+    # [B, Hq, Tq, D] over [B, Tq, Hq, D]
+    return q.bfloat16().cuda().transpose(1, 2), k.bfloat16().cuda()
+
+
+def _select(q, k, **kw):
+    """ids, counts and the workspace bytes the library asked for."""
+    from linattn_amd import _native as N
+    from linattn_amd.kernels.routing import xattn_select_hip
+    lib, seen = N.load(), []
+    orig = lib.la_xattn_select_workspace
+
+    def workspace(a):
+        seen.append(orig(a))
+        return seen[-1]
+
+    lib.la_xattn_select_workspace = workspace
+    try:
+        ids, counts = xattn_select_hip(q, k, **kw)
+    finally:
+        lib.la_xattn_select_workspace = orig
+    return ids, counts, seen[0]
+
+
+def _slot_bytes(shape, n_qb):
+    return shape[0] * shape[1] * n_qb * -(-shape[4] // shape[6]) * 2 * 8
+
+
+@pytest.mark.parametrize("data", ["normal", "few", "wide", "special"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_int8_slots_select_as_fp64(shape, data):
+    B, Hq, Hkv, Tq, T, D, blk, off = shape
+    q, k = _inputs(shape, data)
     for sel in (dict(threshold=0.9), dict(topk=7)):
         kw = dict(block=blk, stride=blk, offset=off, **sel)
-        ids, counts = xattn_select_hip(q, k, **kw)
-        rids, rcounts = xattn_select_hip(q, k, max_workspace_bytes=B * Hq * 64 * n_kb * 2 * 8, **kw)
+        ids, counts, ws = _select(q, k, **kw)
+        # slots of every query block, and the limbs of k and q beside them: the int8 form
+        assert ws > _slot_bytes(shape, -(-Tq // blk)) + 4 * D * B * (Hkv * T + Hq * Tq)
+        rids, rcounts, _ = _select(q, k, max_workspace_bytes=_slot_bytes(shape, 64), **kw)
         assert torch.equal(counts, rcounts)
         assert torch.equal(ids, rids)
+
+
+@pytest.mark.parametrize("data", ["normal", "few", "special"])
+@pytest.mark.parametrize("chunk", [64, 128])
+def test_int8_slots_in_chunks(chunk, data):
+    """Two or three chunks of query blocks, the last one partial (its limbs in buffers
+    laid out for a whole one): the workspace of a call of one chunk's queries is what
+    such a chunk takes, limbs included."""
+    shape = (2, 28, 4, 201 * 4 - 1, 1030, 64, 4, 230)
+    B, Hq, Hkv, Tq, T, D, blk, off = shape
+    q, k = _inputs(shape, data)
+    for sel in (dict(threshold=0.9), dict(topk=7)):
+        kw = dict(block=blk, stride=blk, offset=off, **sel)
+        one = q[:, :, :128 * blk]  # (512 tiles need two rows of them)
+        ws = _select(one, k, **kw)[2]
+        limbs = ws - _slot_bytes(shape, 128)
+        assert limbs > 4 * D * B * (Hkv * T + Hq * 128 * blk)
+        if chunk == 64:  # half the slots, half the limbs of q
+            ws -= _slot_bytes(shape, 64) + 4 * D * B * Hq * 64 * blk
+        ids, counts, full = _select(q, k, max_workspace_bytes=ws, **kw)
+        assert full > ws  # more than one chunk
+        rids, rcounts, _ = _select(q, k, max_workspace_bytes=_slot_bytes(shape, 64), **kw)
+        assert torch.equal(counts, rcounts)
+        assert torch.equal(ids, rids)
+        whole, wcounts, _ = _select(q, k, **kw)
+        assert torch.equal(counts, wcounts) and torch.equal(ids, whole)
 
 
 @pytest.mark.parametrize("data", ["equal", "levels", "normal", "steep"])

@@ -74,8 +74,8 @@ class _Totals:
             return self._host
         if self.captured:
             torch.cuda.synchronize(self.totals.device)
-        else:
-            self.stream.synchronize()
+        elif torch.cuda.current_stream(self.totals.device) != self.stream:
+            self.stream.synchronize()  # (the copy waits for its own stream)
         sums = self.totals.cpu().sum(0).tolist()
         if not self.captured:
             self._host = sums

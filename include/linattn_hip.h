@@ -139,8 +139,10 @@ typedef struct {
  * Work is split over the list ("split-K"); num_splits = 0 picks a split count.
  * With num_splits = 0, calls of many queries over a contiguous bf16 cache
  * (D = 128, bf16 q) run as tiles of queries sharing key blocks when
- * la_sparse_attention_workspace() bytes are given (16-byte aligned); with less,
- * but enough for the split partials, they run row by row.
+ * la_sparse_attention_workspace() bytes are given (16-byte aligned, at most 512
+ * MiB); with less, but enough for the split partials, they run row by row.
+ * out may be q with one split (each row of q is read before that row of out is
+ * written): such calls run row by row.
  */
 typedef struct {
   const void *q;

@@ -14,7 +14,7 @@ struct LrKP {
 
 // 2^lw lanes per row (at least its entries, at most a wave); the same totals as
 // torch's masks and sums over the expanded lists, which took ten launches and two
-// host reads per call: 150 us of a 256-query chunk, about 6 us and no host read
+// host reads per call: 150 us of a 256-query chunk, about 5 us and no host read
 // here.  Every workgroup writes a pair of its own, and the first one zeros the
 // pairs past the grid: sums in one pair took a launch of 3.7 us that cleared it.
 __global__ __launch_bounds__(256) void list_reads_kernel(LrKP p) {

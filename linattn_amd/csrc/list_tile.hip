@@ -572,14 +572,17 @@ static RowCost row_ps(int64_t heads) {
          : heads == 2 ? RowCost{7000.f, 41.f} : RowCost{4000.f, 38.f};
 }
 constexpr float LT_TILE_PS = 1.1f, LT_LEFT_PS = 2000.f;
-// The masks, the merge and the look for marked rows cost about 25 us here, so
-// calls the row kernels finish sooner stay with them (measured, 512 listed
-// tokens per query, 8 heads: 128 queries 34 us by rows, 43 by tiles; 512
-// queries 93 and 50).  The host knows the width of lists, not their counts: wide lists
-// that turn out nearly empty pay those 25 us and the dearer rows (512 queries of 8
+// The masks, the merge and the look for marked rows cost LT_EXTRA_US here, and four
+// launches more on the host, so calls the row kernels finish sooner stay with them:
+// those whose tokens take LT_MIN_ROW_US (512 listed tokens per query, 8 heads: 128
+// queries 34 us by rows, 43 by tiles; 512 queries 93 and 50; 247 queries of 8 lists of
+// 382 tokens for two heads, 3887 keys, 31 us of tokens: a DSA chunk 90 and 95; a window
+// of 260 tokens over 511 keys, 8 heads, 30 us: the variant's prefill, which waits for
+// its host, 126 and 138).  The host knows the width of lists, not their counts: wide lists
+// that turn out nearly empty pay LT_EXTRA_US and the dearer rows (512 queries of 8
 // lists over 8192 keys, units of 8: 1 unit a list 60 us by rows, 72 here, 4 units 62 and
 // 94, 16 units 100 and 130; 64 units 247 and 154, full lists 1400 and 116).
-constexpr float LT_MIN_ROW_US = 40.f;
+constexpr float LT_MIN_ROW_US = 38.f, LT_EXTRA_US = 30.f;
 // Masks, block lists, marks and parts of one call (the row kernels need none of it).
 constexpr size_t LT_MAX_BYTES = (size_t)512 << 20;
 
@@ -629,16 +632,17 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
     return (x * (o + (x + 1) / 2) + (n - x) * cap) / n;
   };
   const RowCost rc = row_ps(per_head ? 1 : G);
-  const double rows_ps = (double)(a->B * a->ids_heads * a->Tq) *
-                         (rc.fixed + rc.tok * mean((double)std::min(a->N * a->unit, kv->T)));
+  const double n_rows = (double)(a->B * a->ids_heads * a->Tq);
+  const double tok_ps = n_rows * rc.tok * mean((double)std::min(a->N * a->unit, kv->T));
+  const double rows_ps = n_rows * rc.fixed + tok_ps;
   const int64_t gt = pow2 ? G : 1, qt = LT_M / gt;
   const double tile_ps = (double)(a->B * (a->Hq / gt) * ceil_div(a->Tq, qt) * LT_M) * LT_TILE_PS * mean((double)kv->T);
-  if (rows_ps < LT_MIN_ROW_US * 1e6) return pl;
+  if (tok_ps < LT_MIN_ROW_US * 1e6) return pl;
   // Surely cheaper: tiles.  Else whole-block lists, whose masks cost little,
   // are looked at tile by tile down to lists of 1/64 of what is within reach
   // (rows that share their blocks: 65536 keys, 17 blocks a row, 64 neighbours
   // drawing from the same 68 blocks: 269 us by rows, 109 by tiles).
-  const bool sure = tile_ps < 0.9 * rows_ps;
+  const bool sure = tile_ps + LT_EXTRA_US * 1e6 < 0.9 * rows_ps;
   if (!sure && (a->unit % LT_BS != 0 || reach > 64 * a->N * a->unit)) return pl;
   pl.sure = sure;
   pl.row_fixed = (rc.fixed + LT_LEFT_PS) / LT_TILE_PS;
@@ -659,7 +663,7 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
   const int64_t tiles = a->B * pl.ngrp * pl.ntile;
   // Nothing to decide where even walking every block beats rows whose counts are 0 (or
   // whose lists, without counts, are walked to the end).
-  const double least_ps = (double)(a->B * a->ids_heads * a->Tq) *
+  const double least_ps = n_rows *
                           (rc.fixed + LT_LEFT_PS + (a->counts ? 0.0 : rc.tok * (double)(a->N * a->unit)));
   pl.decide = !sure ? LT_EACH : tile_ps < LT_LEAVE * least_ps ? LT_TILES
               : tiles <= LT_ONE ? LT_TOGETHER : LT_EACH;

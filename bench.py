@@ -600,7 +600,10 @@ def bench_xattn(dev, steps, warmup):
             "ms_select": round(ms, 4), "blocks_per_row": round(float(counts.float().mean()), 2),
             "frac_causal_blocks_kept": round(int(counts.sum()) / pairs, 4),
             "score_tflops_fp64": round(tflops, 2),
-            "frac_fp64_valu_peak": round(tflops / FP64_VALU_PEAK_TFLOPS, 4)}
+            "frac_fp64_valu_peak": round(tflops / FP64_VALU_PEAK_TFLOPS, 4),
+            "note": "score_tflops_fp64: the exact fp64 slot products over the whole call, scores "
+                    "and selection; bf16 slots are computed exactly as int8 limb products on the "
+                    "matrix cores, so the fraction of the fp64 VALU peak is a scale, not a bound"}
 
 
 def _counter_rows(d):

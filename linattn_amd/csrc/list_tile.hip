@@ -563,7 +563,7 @@ static size_t up256(size_t x) { return (x + 255) / 256 * 256; }
 // LT_TILE_PS for a row and token of a walked block here (0.93-1.06 measured with
 // every CU busy).  A row that its tile leaves costs LT_LEFT_PS more: its workgroup
 // takes several one after another (16384 rows of one head and 32 tokens: 84 us in
-// sparse_attn_mfma_kernel, 108 in sparse_attn_gated_kernel).
+// sparse_attn_mfma_kernel, 106 in sparse_attn_gated_kernel).
 struct RowCost {
   float fixed, tok;
 };
@@ -581,7 +581,8 @@ constexpr float LT_TILE_PS = 1.1f, LT_LEFT_PS = 2000.f;
 // its host, 126 and 138).  The host knows the width of lists, not their counts: wide lists
 // that turn out nearly empty pay LT_EXTRA_US and the dearer rows (512 queries of 8
 // lists over 8192 keys, units of 8: 1 unit a list 60 us by rows, 72 here, 4 units 62 and
-// 94, 16 units 100 and 130; 64 units 247 and 154, full lists 1400 and 116).
+// 94, 16 units 100 and 130; 64 units 247 and 154; 4 units and -1 to the full width,
+// which the row kernel walks, 1418 and 116).
 constexpr float LT_MIN_ROW_US = 38.f, LT_EXTRA_US = 30.f;
 // Masks, block lists, marks and parts of one call (the row kernels need none of it).
 constexpr size_t LT_MAX_BYTES = (size_t)512 << 20;

@@ -778,8 +778,9 @@ __global__ __launch_bounds__(SA_NT, G <= 4 ? 4 : 2) void sparse_attn_mfma_kernel
 // Usually no row is marked and the launch is the look alone.  The merged state of
 // the parts lies in LDS: in registers, held across mfma_attend with all that depends
 // on the lane, four heads spilled 109 of them (49 here, 42 in sparse_attn_mfma_kernel
-// itself).  Every row left, lists of 8 tokens: 4096 rows of four heads 108 us, 65
-// here (60 in sparse_attn_mfma_kernel); 16384 rows of one head 150, 108 (84).
+// itself).  Calls of 512 queries whose every row is left, 32 of 8192 tokens each: 8
+// lists of four heads 137 us, 92 here; 32 lists 196, 131 (this kernel 69 and 106, on
+// sparse_attn_mfma_kernel's 62 and 84).
 template <int G>
 __global__ __launch_bounds__(SA_NT, G <= 4 ? 4 : 2) void sparse_attn_gated_kernel(AttnKP p,
                                                                                   ListTileGate gt,

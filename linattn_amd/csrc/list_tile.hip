@@ -583,7 +583,7 @@ constexpr float LT_TILE_PS = 1.1f, LT_LEFT_PS = 2000.f;
 // lists over 8192 keys, units of 8: 1 unit a list 60 us by rows, 72 here, 4 units 62 and
 // 94, 16 units 100 and 130; 64 units 247 and 154; 4 units and -1 to the full width,
 // which the row kernel walks, 1418 and 116).
-constexpr float LT_MIN_ROW_US = 38.f, LT_EXTRA_US = 30.f;
+constexpr float LT_MIN_ROW_US = 38.f, LT_EXTRA_US = 20.f;
 // Masks, block lists, marks and parts of one call (the row kernels need none of it).
 constexpr size_t LT_MAX_BYTES = (size_t)512 << 20;
 
@@ -643,7 +643,7 @@ ListTilePlan list_tile_plan(const la_sparse_attn_args *a, const la_kv *kv) {
   // are looked at tile by tile down to lists of 1/64 of what is within reach
   // (rows that share their blocks: 65536 keys, 17 blocks a row, 64 neighbours
   // drawing from the same 68 blocks: 269 us by rows, 109 by tiles).
-  const bool sure = tile_ps + LT_EXTRA_US * 1e6 < 0.9 * rows_ps;
+  const bool sure = tile_ps + LT_EXTRA_US * 1e6 < rows_ps;
   if (!sure && (a->unit % LT_BS != 0 || reach > 64 * a->N * a->unit)) return pl;
   pl.sure = sure;
   pl.row_fixed = (rc.fixed + LT_LEFT_PS) / LT_TILE_PS;

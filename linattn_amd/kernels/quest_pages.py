@@ -187,7 +187,8 @@ def quest_select_hip(q: torch.Tensor, mins: torch.Tensor, maxs: torch.Tensor, *,
     union = gqa_union and G > 1
     # (with a position per sequence, two launches would be two per sequence)
     if mins.stride() == maxs.stride() and mins.dtype == maxs.dtype and (
-            union or positions is not None or _heads_in_one_kernel(B * Hq * Tq, P, k, D, G)):
+            (k <= 64 and P <= 256) or union or positions is not None
+            or _heads_in_one_kernel(B * Hq * Tq, P, k, D, G)):
         # one pass: scores and top-k per head, and the union of a group's heads
         heads, width = (Hkv, G * k) if union else (Hq, k)
         ids = torch.empty(B, heads, Tq, width, dtype=torch.int32, device=dev)

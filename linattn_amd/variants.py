@@ -54,10 +54,9 @@ class _Totals:
         shared by every query; listed units are intersected with causality and
         the cache length."""
         B, L, rows, W = ids.shape
-        sb, sh, st = ids.stride(0), ids.stride(1), ids.stride(2)
-        if ids.stride(3) != 1:
+        if ids.stride(-1) != 1:
             ids = ids.contiguous()
-            sb, sh, st = ids.stride(0), ids.stride(1), ids.stride(2)
+        sb, sh, st, _ = ids.stride()
         self.totals = torch.empty(N.LIST_READS_PARTS, 2, dtype=torch.int64, device=ids.device)
         self.stream = torch.cuda.current_stream(ids.device)
         self.captured = torch.cuda.is_current_stream_capturing()
